@@ -33,6 +33,7 @@ HIP_SOURCES = [
     "spmm_cubeop.hip",
     "spmm_rowscalar.hip",
     "preprocess.hip",
+    "preprocess_windows.hip",
 ]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

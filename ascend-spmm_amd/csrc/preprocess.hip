@@ -32,9 +32,11 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <cstring>
 #include <string>
 
 #include "common.h"
+#include "preprocess_windows.h"
 
 namespace spmm {
 namespace pre {
@@ -551,6 +553,9 @@ struct Header {
   int64_t a0, a1, a2, a3;  // pipeline-specific
 };
 constexpr int64_t kMagic = 0x5350'4d4d'5052'4531LL;
+// A plan of the window-by-window pipeline (preprocess_windows.h).
+constexpr int64_t kMagicWindows = 0x5350'4d4d'5052'4532LL;
+static_assert(sizeof(Header) <= sizeof(spmm_plan_record), "a plan record holds the header");
 
 struct TaskState {
   unsigned long long bpos;       // marginal sorted position, or ~0 (none)
@@ -1102,9 +1107,64 @@ void lay_bcsr(Ctx& x, WinSort& S, CubeExtra* cube, const Csr& c, int64_t W, void
   if (cube) cube->lay(x.arena, S.nwin);
 }
 
+// Arrays of the window-by-window pipeline, after the header.
+struct WindowBlocks {
+  Header* header;
+  win::BlockArrays a;
+  size_t used;
+  WindowBlocks(const Csr& c, int64_t W, void* ws) {
+    Arena arena;
+    arena.base = static_cast<char*>(ws);
+    const int64_t nwin = ceil_div(c.rows, W);
+    header = arena.take<Header>(1);
+    a.state = arena.take<win::WindowState>(1);
+    a.nb = arena.take<uint32_t>(nwin);
+    a.ptr = arena.take<uint32_t>(nwin + 1);
+    used = arena.used;
+  }
+};
+
+win::Matrix window_matrix(const Csr& c) {
+  return win::Matrix{c.rows, c.cols, c.nnz, c.it, c.vt, c.rowptr, c.col, c.val};
+}
+
+// Keeps a plan's header: in the caller's record, or at the head of the
+// workspace (synchronises the stream).
+spmm_status store_header(const Header& h, Header* device, spmm_plan_record* record, hipStream_t s) {
+  if (record != nullptr) {
+    std::memcpy(record, &h, sizeof h);
+    return SPMM_OK;
+  }
+  hipError_t e = hipMemcpyAsync(device, &h, sizeof h, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  return check_hip(e, "storing the plan");
+}
+
+spmm_status load_header(Header& h, const Header* device, const spmm_plan_record* record, hipStream_t s) {
+  if (record != nullptr)
+    std::memcpy(&h, record, sizeof h);
+  else if (spmm_status st = read_back(&h, device, 1, s))
+    return st;
+  if (h.magic != kMagic && h.magic != kMagicWindows)
+    return fail(SPMM_ERR_CONTRACT, "workspace does not hold a plan for this call");
+  return SPMM_OK;
+}
+
 template <typename I>
 spmm_status bcsr_plan(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStream_t s,
-                      bool tiles, int64_t* count) {
+                      bool tiles, int64_t* count, spmm_plan_record* record) {
+  const win::Matrix wm = window_matrix(c);
+  if (win::eligible(wm, W)) {
+    const WindowBlocks B(c, W, ws);
+    if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+    if (spmm_status st = win::plan_blocks(wm, W, tiles, B.a, s)) return st;
+    win::WindowState v;
+    if (spmm_status st = read_back(&v, B.a.state, 1, s)) return st;
+    if (v.err == 0) {
+      *count = v.total;
+      return store_header(Header{kMagicWindows, v.p_begin, v.n, v.total, 0, 0, 0, 0}, B.header, record, s);
+    }
+  }
   Ctx x;
   WinSort S;
   CubeExtra cube;
@@ -1123,28 +1183,26 @@ spmm_status bcsr_plan(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStr
   } else {
     *count = S.nb;
   }
-  hipError_t e = hipMemcpyAsync(x.header, &h, sizeof h, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  return check_hip(e, "storing the plan");
-}
-
-spmm_status load_header(Header& h, const Ctx& x) {
-  if (spmm_status st = read_back(&h, x.header, 1, x.stream)) return st;
-  if (h.magic != kMagic) return fail(SPMM_ERR_CONTRACT, "workspace does not hold a plan for this call");
-  return SPMM_OK;
+  return store_header(h, x.header, record, s);
 }
 
 template <typename I>
 spmm_status bcsr_fill(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStream_t s, bool tiles,
-                      void* crow_out, void* uniq_out, void* val_out) {
+                      const spmm_plan_record* record, void* crow_out, void* uniq_out, void* val_out) {
+  if (ws == nullptr || ws_bytes < sizeof(Header)) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+  Header h;
+  if (spmm_status st = load_header(h, static_cast<const Header*>(ws), record, s)) return st;
+  if (h.magic == kMagicWindows) {
+    const WindowBlocks B(c, W, ws);
+    if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+    return win::fill_blocks(window_matrix(c), W, tiles, B.a, crow_out, uniq_out, val_out, s);
+  }
   Ctx x;
   WinSort S;
   CubeExtra cube;
   x.stream = s;
   lay_bcsr(x, S, tiles ? &cube : nullptr, c, W, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
-  Header h;
-  if (spmm_status st = load_header(h, x)) return st;
   S.p_begin = h.p_begin;
   S.n = h.n;
   S.nb = h.nb;
@@ -1308,7 +1366,7 @@ spmm_status hybrid_fill(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipS
   lay_hybrid(x, H, c, W, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
   Header h;
-  if (spmm_status st = load_header(h, x)) return st;
+  if (spmm_status st = load_header(h, x.header, nullptr, x.stream)) return st;
   H.S.p_begin = h.p_begin;
   H.S.n = h.n;
   H.S.nb = h.nb;
@@ -1533,7 +1591,7 @@ spmm_status task_fill(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
   lay_task(x, A, c, layout, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
   Header h;
-  if (spmm_status st = load_header(h, x)) return st;
+  if (spmm_status st = load_header(h, x.header, nullptr, x.stream)) return st;
   WinSort& S = A.S;
   S.p_begin = h.p_begin;
   S.n = h.n;
@@ -1644,48 +1702,79 @@ static spmm_status check_window16(int64_t W, const char* op) {
   return SPMM_OK;
 }
 
-spmm_status spmm_bcsr_plan(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,
-                           int64_t* blocks) {
+}  // extern "C"
+
+// The plan and fill of csr_to_bcsr (tiles false) and csr_to_ascend_cube.
+static spmm_status blocks_plan(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,
+                               bool tiles, int64_t* count, spmm_plan_record* record) {
+  const char* op = tiles ? "csr_to_ascend_cube" : "csr_to_bcsr";
   clear_error();
-  if (spmm_status st = check_matrix(m, "csr_to_bcsr")) return st;
-  if (spmm_status st = check_window16(W, "csr_to_bcsr")) return st;
+  if (spmm_status st = check_matrix(m, op)) return st;
+  if (spmm_status st = check_window16(W, op)) return st;
   const Csr c = from_matrix(m);
   return by_index(c.it, [&](auto i) {
-    return bcsr_plan<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), false, blocks);
+    return bcsr_plan<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), tiles, count, record);
   });
+}
+
+static spmm_status blocks_fill(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, bool tiles,
+                               const spmm_plan_record* record, void* crow, void* uniq, void* value, spmm_stream s) {
+  const char* op = tiles ? "csr_to_ascend_cube" : "csr_to_bcsr";
+  clear_error();
+  if (spmm_status st = check_matrix(m, op)) return st;
+  if (spmm_status st = check_window16(W, op)) return st;
+  const Csr c = from_matrix(m);
+  return by_index(c.it, [&](auto i) {
+    return bcsr_fill<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), tiles, record, crow, uniq, value);
+  });
+}
+
+extern "C" {
+
+spmm_status spmm_bcsr_plan(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,
+                           int64_t* blocks) {
+  return blocks_plan(m, W, ws, ws_bytes, s, false, blocks, nullptr);
 }
 
 spmm_status spmm_bcsr_fill(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, void* crow,
                            void* uniq, void* value, spmm_stream s) {
-  clear_error();
-  if (spmm_status st = check_matrix(m, "csr_to_bcsr")) return st;
-  if (spmm_status st = check_window16(W, "csr_to_bcsr")) return st;
-  const Csr c = from_matrix(m);
-  return by_index(c.it, [&](auto i) {
-    return bcsr_fill<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), false, crow, uniq, value);
-  });
+  return blocks_fill(m, W, ws, ws_bytes, false, nullptr, crow, uniq, value, s);
+}
+
+spmm_status spmm_bcsr_plan_record(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,
+                                  int64_t* blocks, spmm_plan_record* record) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "csr_to_bcsr: null plan record");
+  return blocks_plan(m, W, ws, ws_bytes, s, false, blocks, record);
+}
+
+spmm_status spmm_bcsr_fill_record(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes,
+                                  const spmm_plan_record* record, void* crow, void* uniq, void* value,
+                                  spmm_stream s) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "csr_to_bcsr: null plan record");
+  return blocks_fill(m, W, ws, ws_bytes, false, record, crow, uniq, value, s);
 }
 
 spmm_status spmm_cube_plan(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,
                            int64_t* tiles) {
-  clear_error();
-  if (spmm_status st = check_matrix(m, "csr_to_ascend_cube")) return st;
-  if (spmm_status st = check_window16(W, "csr_to_ascend_cube")) return st;
-  const Csr c = from_matrix(m);
-  return by_index(c.it, [&](auto i) {
-    return bcsr_plan<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), true, tiles);
-  });
+  return blocks_plan(m, W, ws, ws_bytes, s, true, tiles, nullptr);
 }
 
 spmm_status spmm_cube_fill(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, void* crow,
                            void* uniq, void* value, spmm_stream s) {
-  clear_error();
-  if (spmm_status st = check_matrix(m, "csr_to_ascend_cube")) return st;
-  if (spmm_status st = check_window16(W, "csr_to_ascend_cube")) return st;
-  const Csr c = from_matrix(m);
-  return by_index(c.it, [&](auto i) {
-    return bcsr_fill<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), true, crow, uniq, value);
-  });
+  return blocks_fill(m, W, ws, ws_bytes, true, nullptr, crow, uniq, value, s);
+}
+
+spmm_status spmm_cube_plan_record(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,
+                                  int64_t* tiles, spmm_plan_record* record) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "csr_to_ascend_cube: null plan record");
+  return blocks_plan(m, W, ws, ws_bytes, s, true, tiles, record);
+}
+
+spmm_status spmm_cube_fill_record(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes,
+                                  const spmm_plan_record* record, void* crow, void* uniq, void* value,
+                                  spmm_stream s) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "csr_to_ascend_cube: null plan record");
+  return blocks_fill(m, W, ws, ws_bytes, true, record, crow, uniq, value, s);
 }
 
 size_t spmm_hybrid_workspace(const spmm_csr_matrix* m, int64_t W) {

@@ -440,13 +440,14 @@ std::map<std::string, at::Tensor> csr_to_bcsr(at::Tensor crow_ptr, at::Tensor co
   const size_t ws_bytes = spmm_bcsr_workspace(&m, window_size);
   at::Tensor ws = workspace(d.crow, ws_bytes);
   int64_t blocks = 0;
-  raise_status(spmm_bcsr_plan(&m, window_size, ws.data_ptr(), ws_bytes, s, &blocks), "csr_to_bcsr");
+  spmm_plan_record plan;
+  raise_status(spmm_bcsr_plan_record(&m, window_size, ws.data_ptr(), ws_bytes, s, &blocks, &plan), "csr_to_bcsr");
   const int64_t nwin = (nrows + window_size - 1) / window_size;
   std::map<std::string, at::Tensor> out;
   out["crow_window_ptr"] = idx_tensor(d, nwin + 1);
   out["unique_col_ids"] = idx_tensor(d, blocks);
   out["value"] = val_tensor(d, 16 * blocks);
-  raise_status(spmm_bcsr_fill(&m, window_size, ws.data_ptr(), ws_bytes, ptr(out["crow_window_ptr"]),
+  raise_status(spmm_bcsr_fill_record(&m, window_size, ws.data_ptr(), ws_bytes, &plan, ptr(out["crow_window_ptr"]),
                               ptr(out["unique_col_ids"]), ptr(out["value"]), s),
                "csr_to_bcsr");
   return finish(std::move(out), d);
@@ -463,13 +464,15 @@ std::map<std::string, at::Tensor> csr_to_ascend_cube(at::Tensor crow_ptr, at::Te
   const size_t ws_bytes = spmm_cube_workspace(&m, window_size);
   at::Tensor ws = workspace(d.crow, ws_bytes);
   int64_t tiles = 0;
-  raise_status(spmm_cube_plan(&m, window_size, ws.data_ptr(), ws_bytes, s, &tiles), "csr_to_ascend_cube");
+  spmm_plan_record plan;
+  raise_status(spmm_cube_plan_record(&m, window_size, ws.data_ptr(), ws_bytes, s, &tiles, &plan),
+               "csr_to_ascend_cube");
   const int64_t nwin = (nrows + window_size - 1) / window_size;
   std::map<std::string, at::Tensor> out;
   out["crow_window_ptr"] = idx_tensor(d, nwin + 1);
   out["unique_col_ids"] = idx_tensor(d, 16 * tiles);
   out["value"] = val_tensor(d, 256 * tiles);
-  raise_status(spmm_cube_fill(&m, window_size, ws.data_ptr(), ws_bytes, ptr(out["crow_window_ptr"]),
+  raise_status(spmm_cube_fill_record(&m, window_size, ws.data_ptr(), ws_bytes, &plan, ptr(out["crow_window_ptr"]),
                               ptr(out["unique_col_ids"]), ptr(out["value"]), s),
                "csr_to_ascend_cube");
   return finish(std::move(out), d);

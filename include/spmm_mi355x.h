@@ -269,6 +269,15 @@ typedef struct spmm_csr_matrix {
   const void* value;
 } spmm_csr_matrix;
 
+/* A plan's few host-side numbers.  *_plan stores them at the head of the
+ * workspace for its *_fill, which reads them back (a synchronisation each);
+ * *_plan_record returns them to the caller instead, and *_fill_record takes
+ * them, so a conversion synchronises once.  A record goes with the workspace
+ * and the matrix of its plan.  Opaque. */
+typedef struct spmm_plan_record {
+  int64_t words[16];
+} spmm_plan_record;
+
 /* csr_to_bcsr: BCSR(16x1).  Replaces ToBCSR / csr_to_bcsr
  * (extension/custom_op.cpp:594-746).  Outputs: crow_window_ptr[nwin+1],
  * unique_col_ids[blocks], value[16*blocks], nwin = ceil(rows/window_size),
@@ -279,6 +288,13 @@ spmm_status spmm_bcsr_plan(const spmm_csr_matrix* m, int64_t window_size, void* 
 spmm_status spmm_bcsr_fill(const spmm_csr_matrix* m, int64_t window_size, void* workspace,
                            size_t workspace_bytes, void* crow_window_ptr, void* unique_col_ids,
                            void* value, spmm_stream stream);
+spmm_status spmm_bcsr_plan_record(const spmm_csr_matrix* m, int64_t window_size, void* workspace,
+                                  size_t workspace_bytes, spmm_stream stream, int64_t* blocks,
+                                  spmm_plan_record* record);
+spmm_status spmm_bcsr_fill_record(const spmm_csr_matrix* m, int64_t window_size, void* workspace,
+                                  size_t workspace_bytes, const spmm_plan_record* record,
+                                  void* crow_window_ptr, void* unique_col_ids, void* value,
+                                  spmm_stream stream);
 
 /* csr_to_ascend_cube: 16x16 cube tiles.  Replaces your_logic_kernel /
  * csr_to_ascend_cube (extension/custom_op.cpp:429-592).  Outputs:
@@ -290,6 +306,13 @@ spmm_status spmm_cube_plan(const spmm_csr_matrix* m, int64_t window_size, void* 
 spmm_status spmm_cube_fill(const spmm_csr_matrix* m, int64_t window_size, void* workspace,
                            size_t workspace_bytes, void* crow_window_ptr, void* unique_col_ids,
                            void* value, spmm_stream stream);
+spmm_status spmm_cube_plan_record(const spmm_csr_matrix* m, int64_t window_size, void* workspace,
+                                  size_t workspace_bytes, spmm_stream stream, int64_t* tiles,
+                                  spmm_plan_record* record);
+spmm_status spmm_cube_fill_record(const spmm_csr_matrix* m, int64_t window_size, void* workspace,
+                                  size_t workspace_bytes, const spmm_plan_record* record,
+                                  void* crow_window_ptr, void* unique_col_ids, void* value,
+                                  spmm_stream stream);
 
 /* block_level_split: density-threshold BCSR(window_size x 1) + CSR split.
  * Replaces hybrid_split_impl / block_level_split

@@ -1,0 +1,105 @@
+"""The window-by-window preprocessing kernels at the sizes where they change
+behaviour (bitmap word and prefix-group edges, windows longer than the
+registers hold, the LDS tile's edge, the column limit), bit for bit against
+the CPU oracle; and the inputs they hand to the sorting pipeline instead."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from test_gpu_preprocess import assert_same
+
+pytestmark = pytest.mark.gpu
+
+# 31 .. 129: words and prefix groups; 131072 / 131073: 2- and 4-word groups;
+# 524288 / 524289: 4- and 8-word groups; 2^20: the limit; 2^20 + 1: past it.
+COLS = [1, 31, 32, 33, 127, 128, 129, 4097, 131072, 131073, 524288, 524289, 1 << 20, (1 << 20) + 1]
+
+
+def matrix(cols, rows=37, seed=0):
+    """Random short rows, a run of adjacent columns, an empty row, the first
+    and last columns, and one row longer than a work-group holds (4096 or
+    more nonzeros, where there are so many columns)."""
+    rng = np.random.default_rng(cols + seed)
+    parts = [np.unique(rng.integers(0, cols, int(rng.integers(0, 40)))) for _ in range(rows)]
+    parts[2] = np.arange(max(0, cols // 2 - 70), min(cols, cols // 2 + 70))
+    parts[3] = np.zeros(0, np.int64)
+    parts[4] = np.unique(np.array([0, cols - 1]))
+    parts[20] = np.unique(rng.integers(0, cols, min(6 * cols, 9000)))
+    crow = np.zeros(rows + 1, np.int64)
+    crow[1:] = np.cumsum([p.size for p in parts])
+    return crow, np.concatenate(parts).astype(np.int64)
+
+
+def as_types(crow, col, index, value, seed=3):
+    val = np.random.default_rng(seed).uniform(-1, 1, col.size).astype(value)
+    return crow.astype(index), col.astype(index), val
+
+
+def gpu(*arrays):
+    return [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in arrays]
+
+
+@pytest.mark.parametrize("cols", COLS)
+@pytest.mark.parametrize("window", [1, 7, 16])
+def test_blocks_and_tiles(spmm_npu, cols, window):
+    crow, col = matrix(cols)
+    for index, value in ((np.int32, np.float16), (np.int64, np.float32), (np.int32, np.float64)):
+        args = as_types(crow, col, index, value)
+        assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 37, cols, window), O.csr_to_bcsr(*args, 37, cols, window))
+        assert_same(spmm_npu.csr_to_ascend_cube(*gpu(*args), 37, cols, window),
+                    O.csr_to_ascend_cube(*args, 37, cols, window))
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+@pytest.mark.parametrize("blocks,value", [(640, np.float16), (320, np.float32), (160, np.float64)])
+def test_tile_edge(spmm_npu, blocks, value, extra):
+    """A window of exactly as many blocks as the LDS tile holds, one less, one
+    more (20 KB of 16-value blocks)."""
+    n = blocks + extra
+    crow = np.array([0, n, n + 1], np.int64)
+    col = np.concatenate([np.arange(n), [n // 2]]).astype(np.int64)
+    args = as_types(crow, col, np.int32, value)
+    assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 2, 5000, 16), O.csr_to_bcsr(*args, 2, 5000, 16))
+
+
+@pytest.mark.parametrize("n", [4095, 4096, 4097])
+def test_window_of_register_size(spmm_npu, n):
+    """A window of as many nonzeros as a 256-thread work-group holds."""
+    rng = np.random.default_rng(n)
+    rows = [np.sort(rng.choice(3000, k, replace=False)) for k in (1500, n - 3000, 1500)]
+    crow = np.concatenate([[0], np.cumsum([r.size for r in rows])]).astype(np.int64)
+    args = as_types(crow, np.concatenate(rows).astype(np.int64), np.int32, np.float16)
+    assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 3, 3000, 16), O.csr_to_bcsr(*args, 3, 3000, 16))
+
+
+def test_first_position_past_zero(spmm_npu):
+    """A row pointer that starts past the first stored nonzero."""
+    crow, col = matrix(500)
+    crow, col = crow + 11, np.concatenate([np.arange(11), col])
+    args = as_types(crow, col, np.int32, np.float32)
+    assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 37, 500, 16), O.csr_to_bcsr(*args, 37, 500, 16))
+
+
+def test_repeated_and_invalid_columns_take_the_sorting_pipeline(spmm_npu):
+    crow, col = matrix(500)
+    args = as_types(crow, col, np.int32, np.float32)
+    twice = args[1].copy()
+    r = int(np.nonzero(np.diff(crow) > 3)[0][5])
+    twice[crow[r] + 1] = twice[crow[r]]  # the row's second nonzero repeats its first column
+    assert_same(spmm_npu.csr_to_bcsr(*gpu(args[0], twice, args[2]), 37, 500, 16),
+                O.csr_to_bcsr(args[0], twice, args[2], 37, 500, 16))
+    down = args[1].copy()
+    down[crow[r]], down[crow[r] + 1] = args[1][crow[r] + 1], args[1][crow[r]]
+    with pytest.raises(ValueError, match="ascending"):
+        spmm_npu.csr_to_bcsr(*gpu(args[0], down, args[2]), 37, 500, 16)
+    for bad in (500, -1):
+        out = args[1].copy()
+        out[crow[r + 1] - 1 if bad > 0 else crow[r]] = bad
+        with pytest.raises(RuntimeError, match="out of range"):
+            spmm_npu.csr_to_bcsr(*gpu(args[0], out, args[2]), 37, 500, 16)
+    back = args[0].copy()
+    back[r + 1], back[r] = back[r], back[r + 1]
+    with pytest.raises(ValueError, match="row pointer"):
+        spmm_npu.csr_to_bcsr(*gpu(back, args[1], args[2]), 37, 500, 16)
