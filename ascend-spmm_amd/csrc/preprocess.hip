@@ -61,6 +61,20 @@ inline unsigned grid_for(int64_t n) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < (n); \
        i += static_cast<int64_t>(gridDim.x) * blockDim.x)
 
+// preprocess's nine one-element outputs, stored by one launch.
+struct TaskScalars {
+  int64_t ints[6];
+  double doubles[3];
+  int64_t* to_int[6];
+  double* to_double[3];
+};
+__global__ void store_scalars(TaskScalars t) {
+  if (threadIdx.x == 0) {
+    for (int i = 0; i < 6; ++i) *t.to_int[i] = t.ints[i];
+    for (int i = 0; i < 3; ++i) *t.to_double[i] = t.doubles[i];
+  }
+}
+
 // ---------------------------------------------------------------- workspace
 
 // Bump allocator over the caller's workspace.  With base == nullptr it only
@@ -1128,6 +1142,72 @@ win::Matrix window_matrix(const Csr& c) {
   return win::Matrix{c.rows, c.cols, c.nnz, c.it, c.vt, c.rowptr, c.col, c.val};
 }
 
+void lay_window_split(Arena& a, win::SplitArrays& x, int64_t nwin, int64_t nnz, int64_t cols) {
+  x.nb = a.take<uint32_t>(nwin);
+  x.hist = a.take<uint32_t>(16 * nwin);
+  x.total = a.take<uint32_t>(16 * win::kHistCopies);
+  x.moved = a.take<uint32_t>(nwin);
+  x.kptr = a.take<uint32_t>(nwin + 1);
+  x.vptr = a.take<uint32_t>(nwin + 1);
+  x.occ = a.take<uint32_t>(nnz);
+  x.first = a.take<uint32_t>(std::min(nnz, cols));
+  x.rule = a.take<uint32_t>(1);
+}
+
+struct WindowSplit {
+  Header* header;
+  win::WindowState* state;
+  win::SplitArrays x;
+  size_t used;
+  WindowSplit(const Csr& c, int64_t W, void* ws) {
+    Arena arena;
+    arena.base = static_cast<char*>(ws);
+    header = arena.take<Header>(1);
+    state = arena.take<win::WindowState>(1);
+    lay_window_split(arena, x, ceil_div(c.rows, W), c.nnz, c.cols);
+    used = arena.used;
+  }
+};
+
+struct WindowTask {
+  Header* header;
+  win::TaskArrays x;
+  size_t used;
+  WindowTask(const Csr& c, bool layout, void* ws) {
+    Arena a;
+    a.base = static_cast<char*>(ws);
+    const int64_t nwin = ceil_div(c.rows, 16), m = std::min(c.nnz, c.cols);
+    header = a.take<Header>(1);
+    x.record = a.take<win::TaskRecord>(1);
+    x.nb = a.take<uint32_t>(nwin);
+    x.dkey = a.take<uint64_t>(nwin);
+    x.sdkey = a.take<uint64_t>(nwin);
+    x.wid = a.take<uint32_t>(nwin);
+    x.rank = a.take<uint32_t>(nwin);
+    x.swin = a.take<uint32_t>(nwin);
+    x.sbz = a.take<uint64_t>(nwin);
+    x.pnb = a.take<uint32_t>(nwin + 1);
+    x.pnnz = a.take<uint32_t>(nwin + 1);
+    x.mocc = a.take<uint32_t>(m);
+    x.mfirst = a.take<uint32_t>(m);
+    x.midx = a.take<uint32_t>(m);
+    x.mrow = a.take<uint32_t>(17);
+    x.temp_bytes = win::task_temp_bytes(win::Matrix{c.rows, c.cols, c.nnz, c.it, c.vt, c.rowptr, c.col, c.val}, layout);
+    x.temp = a.take<char>(static_cast<int64_t>(x.temp_bytes));
+    x.split = win::SplitArrays{};
+    if (layout) {
+      x.inv = a.take<uint32_t>(c.rows);
+      x.tkey = a.take<uint32_t>(c.nnz);
+      x.stkey = a.take<uint32_t>(c.nnz);
+      x.tword = a.take<uint64_t>(c.nnz);
+      x.stword = a.take<uint64_t>(c.nnz);
+      x.rp = a.take<uint32_t>(16 * nwin + 1);
+      lay_window_split(a, x.split, nwin, c.nnz, 16 * nwin);
+    }
+    used = a.used;
+  }
+};
+
 // Keeps a plan's header: in the caller's record, or at the head of the
 // workspace (synchronises the stream).
 spmm_status store_header(const Header& h, Header* device, spmm_plan_record* record, hipStream_t s) {
@@ -1343,7 +1423,20 @@ void lay_hybrid(Ctx& x, HybridArrays& H, const Csr& c, int64_t W, void* ws) {
 
 template <typename I>
 spmm_status hybrid_plan(const Csr& c, double a, int64_t W, void* ws, size_t ws_bytes, hipStream_t s,
-                        int64_t* kept, int64_t* vnnz) {
+                        int64_t* kept, int64_t* vnnz, spmm_plan_record* record) {
+  const win::Matrix wm = window_matrix(c);
+  if (win::eligible(wm, W)) {
+    const WindowSplit B(c, W, ws);
+    if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+    if (spmm_status st = win::plan_split(wm, a, W, B.x, B.state, s)) return st;
+    win::WindowState v;
+    if (spmm_status st = read_back(&v, B.state, 1, s)) return st;
+    if (v.err == 0) {
+      *kept = v.total;
+      *vnnz = v.vnnz;
+      return store_header(Header{kMagicWindows, 0, 0, 0, v.total, v.vnnz, 0, 0}, B.header, record, s);
+    }
+  }
   Ctx x;
   HybridArrays H;
   x.stream = s;
@@ -1351,22 +1444,26 @@ spmm_status hybrid_plan(const Csr& c, double a, int64_t W, void* ws, size_t ws_b
   lay_hybrid(x, H, c, W, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
   if (spmm_status st = hybrid_run<I>(c, a, W, H, x, kept, vnnz)) return st;
-  Header h{kMagic, H.S.p_begin, H.S.n, H.S.nb, *kept, *vnnz, 0, 0};
-  hipError_t e = hipMemcpyAsync(x.header, &h, sizeof h, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  return check_hip(e, "storing the plan");
+  return store_header(Header{kMagic, H.S.p_begin, H.S.n, H.S.nb, *kept, *vnnz, 0, 0}, x.header, record, s);
 }
 
 template <typename I>
-spmm_status hybrid_fill(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStream_t s, void* crow,
-                        void* uniq, void* val, void* vrow, void* vcol, void* vval) {
+spmm_status hybrid_fill(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStream_t s,
+                        const spmm_plan_record* record, void* crow, void* uniq, void* val, void* vrow, void* vcol,
+                        void* vval) {
+  if (ws == nullptr || ws_bytes < sizeof(Header)) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+  Header h;
+  if (spmm_status st = load_header(h, static_cast<const Header*>(ws), record, s)) return st;
+  if (h.magic == kMagicWindows) {
+    const WindowSplit B(c, W, ws);
+    if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+    return win::fill_split(window_matrix(c), W, B.x, crow, uniq, val, vrow, vcol, vval, s);
+  }
   Ctx x;
   HybridArrays H;
   x.stream = s;
   lay_hybrid(x, H, c, W, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
-  Header h;
-  if (spmm_status st = load_header(h, x.header, nullptr, x.stream)) return st;
   H.S.p_begin = h.p_begin;
   H.S.n = h.n;
   H.S.nb = h.nb;
@@ -1453,13 +1550,52 @@ void lay_task(Ctx& x, TaskArrays& A, const Csr& c, bool layout, void* ws) {
   A.lay(x.arena, c, layout);
 }
 
+// The window-by-window pipeline takes the matrix, and its transpose's columns
+// (packed rows) too where the graph layout asks for it.
+bool window_task_eligible(const Csr& c, bool graph_layout) {
+  return win::eligible(window_matrix(c), 16) &&
+         (!(graph_layout && c.rows == c.cols) || 16 * ceil_div(c.rows, 16) <= win::kMaxColumns);
+}
+
 Csr transposed_csr(const Csr& c, const TaskArrays& A, int64_t out_rows, int64_t n) {
   return Csr{out_rows, out_rows, n, SPMM_INDEX_I64, c.vt, A.rpT, A.colT, A.valT};
 }
 
 template <typename I>
 spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes, hipStream_t s,
-                      spmm_taskmap_info* info) {
+                      spmm_taskmap_info* info, spmm_plan_record* record) {
+  const win::Matrix wm = window_matrix(c);
+  if (window_task_eligible(c, graph_layout)) {
+    const bool layout = graph_layout && c.rows == c.cols;
+    const WindowTask B(c, layout, ws);
+    if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+    if (spmm_status st = win::plan_task(wm, layout, B.x, s)) return st;
+    win::TaskRecord v;
+    if (spmm_status st = read_back(&v, B.x.record, 1, s)) return st;
+    if (v.err == 0) {
+      spmm_taskmap_info r{};
+      r.aic_windows = v.naic;
+      r.aic_blocks = v.aic_blocks;
+      r.packed_rows = v.out_rows;
+      r.vector_nnz = v.vnnz;
+      r.packed_layout_supported = layout ? 1 : 0;
+      r.marginal_window = v.bwin;
+      r.marginal_aic_blocks = v.baic;
+      r.marginal_total_blocks = v.bblocks;
+      r.shared_windows = v.shared;
+      r.estimated_aic_cost = v.est_aic;
+      r.estimated_aiv_cost = v.est_aiv;
+      r.estimated_max_cost = v.est_max;
+      if (layout) {
+        r.t_windows = ceil_div(c.rows, 16);
+        r.t_blocks = v.t_kept;
+        r.t_rows = 16 * r.t_windows;
+        r.t_vector_nnz = v.t_vnnz;
+      }
+      *info = r;
+      return store_header(Header{kMagicWindows, v.p_begin, v.n, 0, 0, 0, 0, v.naic}, B.header, record, s);
+    }
+  }
   Ctx x;
   TaskArrays A;
   x.stream = s;
@@ -1573,25 +1709,34 @@ spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
     r.t_vector_nnz = tv;
   }
   *info = r;
-  if (!layout) return SPMM_OK;  // collect_taskmap stored the plan header
+  // collect_taskmap stored the plan header; a record takes the same numbers.
+  if (record != nullptr) {
+    const Header h{kMagic, S.p_begin, n, nb, aic_blocks, vnnz, hs.out_rows, hs.naic};
+    std::memcpy(record, &h, sizeof h);
+  }
+  if (!layout) return SPMM_OK;
   // The transpose split's sizes beside it.
-  Header ht{kMagic, A.T.S.p_begin, A.T.S.n, A.T.S.nb, r.t_blocks, r.t_vector_nnz, 0, 0};
-  hipError_t e = hipMemcpyAsync(A.theader, &ht, sizeof ht, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  return check_hip(e, "storing the plan");
+  return store_header(Header{kMagic, A.T.S.p_begin, A.T.S.n, A.T.S.nb, r.t_blocks, r.t_vector_nnz, 0, 0}, A.theader,
+                      nullptr, s);
 }
 
 template <typename I>
 spmm_status task_fill(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes, hipStream_t s,
-                      const spmm_taskmap_out* o) {
+                      const spmm_plan_record* record, const spmm_taskmap_out* o) {
+  if (ws == nullptr || ws_bytes < sizeof(Header)) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+  Header h;
+  if (spmm_status st = load_header(h, static_cast<const Header*>(ws), record, s)) return st;
+  if (h.magic == kMagicWindows) {
+    const WindowTask B(c, graph_layout && c.rows == c.cols, ws);
+    if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
+    return win::fill_task(window_matrix(c), graph_layout && c.rows == c.cols, h.a3, B.x, o, s);
+  }
   Ctx x;
   TaskArrays A;
   x.stream = s;
   const bool layout = graph_layout && c.rows == c.cols;
   lay_task(x, A, c, layout, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
-  Header h;
-  if (spmm_status st = load_header(h, x.header, nullptr, x.stream)) return st;
   WinSort& S = A.S;
   S.p_begin = h.p_begin;
   S.n = h.n;
@@ -1672,8 +1817,9 @@ size_t bcsr_bytes(const spmm_csr_matrix* m, int64_t W, bool tiles) {
   Ctx x;
   WinSort S;
   CubeExtra cube;
-  lay_bcsr(x, S, tiles ? &cube : nullptr, from_matrix(m), W, nullptr);
-  return x.arena.used;
+  const Csr c = from_matrix(m);
+  lay_bcsr(x, S, tiles ? &cube : nullptr, c, W, nullptr);
+  return win::eligible(window_matrix(c), W) ? std::max(x.arena.used, WindowBlocks(c, W, nullptr).used) : x.arena.used;
 }
 
 }  // namespace
@@ -1781,32 +1927,57 @@ size_t spmm_hybrid_workspace(const spmm_csr_matrix* m, int64_t W) {
   if (m == nullptr || W < 1) return 0;
   Ctx x;
   HybridArrays H;
-  lay_hybrid(x, H, from_matrix(m), W, nullptr);
-  return x.arena.used;
+  const Csr c = from_matrix(m);
+  lay_hybrid(x, H, c, W, nullptr);
+  return win::eligible(window_matrix(c), W) ? std::max(x.arena.used, WindowSplit(c, W, nullptr).used) : x.arena.used;
 }
 
-spmm_status spmm_hybrid_plan(const spmm_csr_matrix* m, double a, int64_t W, void* ws, size_t ws_bytes,
-                             spmm_stream s, int64_t* kept, int64_t* vnnz) {
+static spmm_status split_plan(const spmm_csr_matrix* m, double a, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,
+                              int64_t* kept, int64_t* vnnz, spmm_plan_record* record) {
   clear_error();
   if (spmm_status st = check_matrix(m, "block_level_split")) return st;
   if (W < 1) return fail(SPMM_ERR_INVALID_ARGUMENT, "block_level_split: window_size must be positive");
   const Csr c = from_matrix(m);
   return by_index(c.it, [&](auto i) {
-    return hybrid_plan<decltype(i)>(c, a, W, ws, ws_bytes, as_stream(s), kept, vnnz);
+    return hybrid_plan<decltype(i)>(c, a, W, ws, ws_bytes, as_stream(s), kept, vnnz, record);
   });
+}
+
+static spmm_status split_fill(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes,
+                              const spmm_plan_record* record, void* crow, void* uniq, void* value, void* vrow,
+                              void* vcol, void* vval, spmm_stream s) {
+  clear_error();
+  if (spmm_status st = check_matrix(m, "block_level_split")) return st;
+  if (W < 1) return fail(SPMM_ERR_INVALID_ARGUMENT, "block_level_split: window_size must be positive");
+  const Csr c = from_matrix(m);
+  return by_index(c.it, [&](auto i) {
+    return hybrid_fill<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), record, crow, uniq, value, vrow, vcol, vval);
+  });
+}
+
+spmm_status spmm_hybrid_plan(const spmm_csr_matrix* m, double a, int64_t W, void* ws, size_t ws_bytes,
+                             spmm_stream s, int64_t* kept, int64_t* vnnz) {
+  return split_plan(m, a, W, ws, ws_bytes, s, kept, vnnz, nullptr);
 }
 
 spmm_status spmm_hybrid_fill(const spmm_csr_matrix* m, double a, int64_t W, void* ws, size_t ws_bytes,
                              void* crow, void* uniq, void* value, void* vrow, void* vcol, void* vval,
                              spmm_stream s) {
-  clear_error();
   (void)a;
-  if (spmm_status st = check_matrix(m, "block_level_split")) return st;
-  if (W < 1) return fail(SPMM_ERR_INVALID_ARGUMENT, "block_level_split: window_size must be positive");
-  const Csr c = from_matrix(m);
-  return by_index(c.it, [&](auto i) {
-    return hybrid_fill<decltype(i)>(c, W, ws, ws_bytes, as_stream(s), crow, uniq, value, vrow, vcol, vval);
-  });
+  return split_fill(m, W, ws, ws_bytes, nullptr, crow, uniq, value, vrow, vcol, vval, s);
+}
+
+spmm_status spmm_hybrid_plan_record(const spmm_csr_matrix* m, double a, int64_t W, void* ws, size_t ws_bytes,
+                                    spmm_stream s, int64_t* kept, int64_t* vnnz, spmm_plan_record* record) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "block_level_split: null plan record");
+  return split_plan(m, a, W, ws, ws_bytes, s, kept, vnnz, record);
+}
+
+spmm_status spmm_hybrid_fill_record(const spmm_csr_matrix* m, int64_t W, void* ws, size_t ws_bytes,
+                                    const spmm_plan_record* record, void* crow, void* uniq, void* value, void* vrow,
+                                    void* vcol, void* vval, spmm_stream s) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "block_level_split: null plan record");
+  return split_fill(m, W, ws, ws_bytes, record, crow, uniq, value, vrow, vcol, vval, s);
 }
 
 size_t spmm_taskmap_workspace(const spmm_csr_matrix* m, int64_t W, int graph_layout) {
@@ -1814,32 +1985,74 @@ size_t spmm_taskmap_workspace(const spmm_csr_matrix* m, int64_t W, int graph_lay
   Ctx x;
   TaskArrays A;
   const Csr c = from_matrix(m);
-  lay_task(x, A, c, graph_layout && c.rows == c.cols, nullptr);
-  return x.arena.used;
+  const bool layout = graph_layout && c.rows == c.cols;
+  lay_task(x, A, c, layout, nullptr);
+  return window_task_eligible(c, graph_layout != 0) ? std::max(x.arena.used, WindowTask(c, layout, nullptr).used)
+                                                    : x.arena.used;
 }
 
-spmm_status spmm_taskmap_plan(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws,
-                              size_t ws_bytes, spmm_stream s, spmm_taskmap_info* info) {
+static spmm_status mapping_plan(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws, size_t ws_bytes,
+                                spmm_stream s, spmm_taskmap_info* info, spmm_plan_record* record) {
   clear_error();
   if (spmm_status st = check_matrix(m, "preprocess")) return st;
   if (W != 16) return fail(SPMM_ERR_CONTRACT, "Ascend-SpMM requires a 16-row window");
   if (info == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "preprocess: null info");
   const Csr c = from_matrix(m);
   return by_index(c.it, [&](auto i) {
-    return task_plan<decltype(i)>(c, graph_layout != 0, ws, ws_bytes, as_stream(s), info);
+    return task_plan<decltype(i)>(c, graph_layout != 0, ws, ws_bytes, as_stream(s), info, record);
   });
 }
 
-spmm_status spmm_taskmap_fill(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws,
-                              size_t ws_bytes, const spmm_taskmap_out* out, spmm_stream s) {
+static spmm_status mapping_fill(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws, size_t ws_bytes,
+                                const spmm_plan_record* record, const spmm_taskmap_out* out, spmm_stream s) {
   clear_error();
   if (spmm_status st = check_matrix(m, "preprocess")) return st;
   if (W != 16) return fail(SPMM_ERR_CONTRACT, "Ascend-SpMM requires a 16-row window");
   if (out == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "preprocess: null outputs");
   const Csr c = from_matrix(m);
   return by_index(c.it, [&](auto i) {
-    return task_fill<decltype(i)>(c, graph_layout != 0, ws, ws_bytes, as_stream(s), out);
+    return task_fill<decltype(i)>(c, graph_layout != 0, ws, ws_bytes, as_stream(s), record, out);
   });
+}
+
+spmm_status spmm_taskmap_plan(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws,
+                              size_t ws_bytes, spmm_stream s, spmm_taskmap_info* info) {
+  return mapping_plan(m, W, graph_layout, ws, ws_bytes, s, info, nullptr);
+}
+
+spmm_status spmm_taskmap_fill(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws,
+                              size_t ws_bytes, const spmm_taskmap_out* out, spmm_stream s) {
+  return mapping_fill(m, W, graph_layout, ws, ws_bytes, nullptr, out, s);
+}
+
+spmm_status spmm_taskmap_plan_record(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws,
+                                     size_t ws_bytes, spmm_stream s, spmm_taskmap_info* info,
+                                     spmm_plan_record* record) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "preprocess: null plan record");
+  return mapping_plan(m, W, graph_layout, ws, ws_bytes, s, info, record);
+}
+
+spmm_status spmm_taskmap_fill_record(const spmm_csr_matrix* m, int64_t W, int graph_layout, void* ws,
+                                     size_t ws_bytes, const spmm_plan_record* record, const spmm_taskmap_out* out,
+                                     spmm_stream s) {
+  if (record == nullptr) return fail(SPMM_ERR_INVALID_ARGUMENT, "preprocess: null plan record");
+  return mapping_fill(m, W, graph_layout, ws, ws_bytes, record, out, s);
+}
+
+spmm_status spmm_taskmap_scalars(const spmm_taskmap_info* info, int64_t* const* ints, double* const* doubles,
+                                 spmm_stream s) {
+  clear_error();
+  if (info == nullptr || ints == nullptr || doubles == nullptr)
+    return fail(SPMM_ERR_INVALID_ARGUMENT, "preprocess: null scalars");
+  TaskScalars t{{info->packed_rows, info->packed_layout_supported, info->marginal_window, info->marginal_aic_blocks,
+                 info->marginal_total_blocks, info->shared_windows},
+                {info->estimated_aic_cost, info->estimated_aiv_cost, info->estimated_max_cost},
+                {},
+                {}};
+  for (int i = 0; i < 6; ++i) t.to_int[i] = ints[i];
+  for (int i = 0; i < 3; ++i) t.to_double[i] = doubles[i];
+  hipLaunchKernelGGL(store_scalars, dim3(1), dim3(64), 0, as_stream(s), t);
+  return check_launch("store_scalars");
 }
 
 }  // extern "C"

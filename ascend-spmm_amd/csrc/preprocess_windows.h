@@ -45,6 +45,65 @@ struct BlockArrays {
   uint32_t* ptr;  // [nwin + 1] exclusive sums
 };
 
+// preprocess (16-row windows).  Device record of its plan.
+struct TaskRecord {
+  int64_t err;
+  int64_t p_begin, n;
+  int64_t bpos;            // sorted position of the marginal window, -1: none
+  int64_t bwin, bblocks;   // the marginal window and its blocks
+  int64_t baic, shared;    // its blocks on the block part; both parts hold some
+  int64_t naic;            // windows of the block part
+  int64_t aic_blocks, vnnz, shared_nnz;
+  int64_t last_pos;        // sorted position of the last (perhaps shorter) window
+  int64_t out_rows;
+  double est_aic, est_aiv, est_max;
+  int64_t t_kept, t_vnnz;  // graph layout: the transpose's split
+};
+
+// block_level_split, and the graph layout's transpose.
+struct SplitArrays {
+  uint32_t* nb;     // [nwin] blocks per window
+  uint32_t* hist;   // [16][nwin] blocks by occupancy
+  uint32_t* total;  // [kHistCopies][16] sums of hist over the windows, in copies
+  uint32_t* moved;  // [nwin] blocks of the boundary occupancy that move
+  uint32_t* kptr;   // [nwin + 1] kept blocks before
+  uint32_t* vptr;   // [nwin + 1] moved nonzeros before
+  uint32_t* occ;    // [nnz] occupancies of windows too wide for LDS
+  uint32_t* first;  // [min(nnz, cols)] first nonzeros of the boundary window's blocks
+  uint32_t* rule;   // [1] boundary occupancy
+};
+constexpr int kHistCopies = 64;
+
+spmm_status plan_split(const Matrix& m, double a, int64_t W, const SplitArrays& x, WindowState* state, hipStream_t s);
+spmm_status fill_split(const Matrix& m, int64_t W, const SplitArrays& x, void* crow, void* uniq, void* val, void* vrow,
+                       void* vcol, void* vval, hipStream_t s);
+
+struct TaskArrays {
+  TaskRecord* record;
+  uint32_t* nb;        // [nwin]
+  uint64_t *dkey, *sdkey;
+  uint32_t *wid, *rank, *swin;  // windows, their ranks and order by density
+  uint64_t* sbz;         // [nwin] blocks << 32 | nonzeros, in that order
+  uint32_t *pnb, *pnnz;  // [nwin + 1] blocks and nonzeros before, in that order
+  uint32_t *mocc, *mfirst, *midx;  // [min(nnz, cols)] marginal window's blocks
+  uint32_t* mrow;                  // [17]
+  void* temp;
+  size_t temp_bytes;
+  // graph layout
+  uint32_t* inv;               // [rows]
+  uint32_t *tkey, *stkey;      // [nnz] packed row of each transposed entry
+  uint64_t *tword, *stword;    // [nnz] packed column << 32 | value bits (or entry)
+  uint32_t* rp;                // [16 nwin + 1] transposed row pointer
+  SplitArrays split;
+};
+
+// Temporary bytes of the device sorts.
+size_t task_temp_bytes(const Matrix& m, bool layout);
+spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, hipStream_t s);
+// naic: the plan's TaskRecord::naic.
+spmm_status fill_task(const Matrix& m, bool layout, int64_t naic, const TaskArrays& x, const spmm_taskmap_out* o,
+                      hipStream_t s);
+
 spmm_status plan_blocks(const Matrix& m, int64_t W, bool tiles, const BlockArrays& a, hipStream_t s);
 spmm_status fill_blocks(const Matrix& m, int64_t W, bool tiles, const BlockArrays& a, void* crow, void* uniq,
                         void* val, hipStream_t s);

@@ -448,7 +448,7 @@ std::map<std::string, at::Tensor> csr_to_bcsr(at::Tensor crow_ptr, at::Tensor co
   out["unique_col_ids"] = idx_tensor(d, blocks);
   out["value"] = val_tensor(d, 16 * blocks);
   raise_status(spmm_bcsr_fill_record(&m, window_size, ws.data_ptr(), ws_bytes, &plan, ptr(out["crow_window_ptr"]),
-                              ptr(out["unique_col_ids"]), ptr(out["value"]), s),
+                                     ptr(out["unique_col_ids"]), ptr(out["value"]), s),
                "csr_to_bcsr");
   return finish(std::move(out), d);
 }
@@ -489,7 +489,8 @@ std::map<std::string, at::Tensor> block_level_split(at::Tensor crow_ptr, at::Ten
   const size_t ws_bytes = spmm_hybrid_workspace(&m, window_size);
   at::Tensor ws = workspace(d.crow, ws_bytes);
   int64_t kept = 0, vnnz = 0;
-  raise_status(spmm_hybrid_plan(&m, a, window_size, ws.data_ptr(), ws_bytes, s, &kept, &vnnz),
+  spmm_plan_record plan;
+  raise_status(spmm_hybrid_plan_record(&m, a, window_size, ws.data_ptr(), ws_bytes, s, &kept, &vnnz, &plan),
                "block_level_split");
   const int64_t nwin = window_size > 0 ? (nrows + window_size - 1) / window_size : 0;
   std::map<std::string, at::Tensor> out;
@@ -499,9 +500,9 @@ std::map<std::string, at::Tensor> block_level_split(at::Tensor crow_ptr, at::Ten
   out["vrow_window_ptr"] = idx_tensor(d, nwin * window_size + 1);
   out["vcol_indices"] = idx_tensor(d, vnnz);
   out["vvalue"] = val_tensor(d, vnnz);
-  raise_status(spmm_hybrid_fill(&m, a, window_size, ws.data_ptr(), ws_bytes, ptr(out["crow_window_ptr"]),
-                                ptr(out["unique_col_ids"]), ptr(out["value"]), ptr(out["vrow_window_ptr"]),
-                                ptr(out["vcol_indices"]), ptr(out["vvalue"]), s),
+  raise_status(spmm_hybrid_fill_record(&m, window_size, ws.data_ptr(), ws_bytes, &plan, ptr(out["crow_window_ptr"]),
+                                       ptr(out["unique_col_ids"]), ptr(out["value"]), ptr(out["vrow_window_ptr"]),
+                                       ptr(out["vcol_indices"]), ptr(out["vvalue"]), s),
                "block_level_split");
   return finish(std::move(out), d);
 }
@@ -518,7 +519,8 @@ std::map<std::string, at::Tensor> preprocess(at::Tensor crow_ptr, at::Tensor col
   const size_t ws_bytes = spmm_taskmap_workspace(&m, window_size, graph_layout ? 1 : 0);
   at::Tensor ws = workspace(d.crow, ws_bytes);
   spmm_taskmap_info info;
-  raise_status(spmm_taskmap_plan(&m, window_size, graph_layout ? 1 : 0, ws.data_ptr(), ws_bytes, s, &info),
+  spmm_plan_record plan;
+  raise_status(spmm_taskmap_plan_record(&m, window_size, graph_layout ? 1 : 0, ws.data_ptr(), ws_bytes, s, &info, &plan),
                "preprocess");
   const bool layout = info.packed_layout_supported != 0;
   std::map<std::string, at::Tensor> out;
@@ -556,19 +558,25 @@ std::map<std::string, at::Tensor> preprocess(at::Tensor crow_ptr, at::Tensor col
   o.transpose_vvalue = ptr(out["transpose_vvalue"]);
   o.permutation = static_cast<int64_t*>(ptr(out["permutation"]));
   o.inv_permutation = static_cast<int64_t*>(ptr(out["inv_permutation"]));
-  raise_status(spmm_taskmap_fill(&m, window_size, graph_layout ? 1 : 0, ws.data_ptr(), ws_bytes, &o, s),
+  raise_status(spmm_taskmap_fill_record(&m, window_size, graph_layout ? 1 : 0, ws.data_ptr(), ws_bytes, &plan, &o, s),
                "preprocess");
-  auto scalar = [&](int64_t v) { return at::full({1}, v, i64); };
-  auto dscalar = [&](double v) { return at::full({1}, v, d.crow.options().dtype(at::kDouble)); };
-  out["packed_rows"] = scalar(info.packed_rows);
-  out["packed_layout_supported"] = scalar(info.packed_layout_supported);
-  out["marginal_window"] = scalar(info.marginal_window);
-  out["marginal_aic_blocks"] = scalar(info.marginal_aic_blocks);
-  out["marginal_total_blocks"] = scalar(info.marginal_total_blocks);
-  out["estimated_aic_cost"] = dscalar(info.estimated_aic_cost);
-  out["estimated_aiv_cost"] = dscalar(info.estimated_aiv_cost);
-  out["estimated_max_cost"] = dscalar(info.estimated_max_cost);
-  out["shared_windows"] = scalar(info.shared_windows);
+  // One-element outputs, stored by one launch.
+  const char* const int_keys[6] = {"packed_rows", "packed_layout_supported", "marginal_window",
+                                   "marginal_aic_blocks", "marginal_total_blocks", "shared_windows"};
+  const char* const double_keys[3] = {"estimated_aic_cost", "estimated_aiv_cost", "estimated_max_cost"};
+  int64_t* ints[6];
+  double* doubles[3];
+  for (int i = 0; i < 6; ++i) {
+    at::Tensor t = at::empty({1}, i64);
+    ints[i] = t.data_ptr<int64_t>();
+    out[int_keys[i]] = t;
+  }
+  for (int i = 0; i < 3; ++i) {
+    at::Tensor t = at::empty({1}, d.crow.options().dtype(at::kDouble));
+    doubles[i] = t.data_ptr<double>();
+    out[double_keys[i]] = t;
+  }
+  raise_status(spmm_taskmap_scalars(&info, ints, doubles, s), "preprocess");
   return finish(std::move(out), d);
 }
 

@@ -328,6 +328,15 @@ spmm_status spmm_hybrid_fill(const spmm_csr_matrix* m, double a, int64_t window_
                              void* workspace, size_t workspace_bytes, void* crow_window_ptr,
                              void* unique_col_ids, void* value, void* vrow_window_ptr,
                              void* vcol_indices, void* vvalue, spmm_stream stream);
+spmm_status spmm_hybrid_plan_record(const spmm_csr_matrix* m, double a, int64_t window_size,
+                                    void* workspace, size_t workspace_bytes, spmm_stream stream,
+                                    int64_t* kept_blocks, int64_t* vector_nnz,
+                                    spmm_plan_record* record);
+spmm_status spmm_hybrid_fill_record(const spmm_csr_matrix* m, int64_t window_size, void* workspace,
+                                    size_t workspace_bytes, const spmm_plan_record* record,
+                                    void* crow_window_ptr, void* unique_col_ids, void* value,
+                                    void* vrow_window_ptr, void* vcol_indices, void* vvalue,
+                                    spmm_stream stream);
 
 /* preprocess: the 295/505 cost-model AIC/AIV task mapping with the marginal
  * window split, row permutation and (graph_layout on a square matrix) the
@@ -381,6 +390,21 @@ spmm_status spmm_taskmap_plan(const spmm_csr_matrix* m, int64_t window_size, int
 spmm_status spmm_taskmap_fill(const spmm_csr_matrix* m, int64_t window_size, int graph_layout,
                               void* workspace, size_t workspace_bytes,
                               const spmm_taskmap_out* out, spmm_stream stream);
+spmm_status spmm_taskmap_plan_record(const spmm_csr_matrix* m, int64_t window_size,
+                                     int graph_layout, void* workspace, size_t workspace_bytes,
+                                     spmm_stream stream, spmm_taskmap_info* info,
+                                     spmm_plan_record* record);
+spmm_status spmm_taskmap_fill_record(const spmm_csr_matrix* m, int64_t window_size,
+                                     int graph_layout, void* workspace, size_t workspace_bytes,
+                                     const spmm_plan_record* record, const spmm_taskmap_out* out,
+                                     spmm_stream stream);
+
+/* Stores info's numbers in one launch, each to a device buffer of one element:
+ * ints = packed_rows, packed_layout_supported, marginal_window,
+ * marginal_aic_blocks, marginal_total_blocks, shared_windows; doubles =
+ * estimated aic, aiv and max cost. */
+spmm_status spmm_taskmap_scalars(const spmm_taskmap_info* info, int64_t* const* ints,
+                                 double* const* doubles, spmm_stream stream);
 
 #ifdef __cplusplus
 }  /* extern "C" */

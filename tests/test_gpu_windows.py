@@ -103,3 +103,89 @@ def test_repeated_and_invalid_columns_take_the_sorting_pipeline(spmm_npu):
     back[r + 1], back[r] = back[r], back[r + 1]
     with pytest.raises(ValueError, match="row pointer"):
         spmm_npu.csr_to_bcsr(*gpu(back, args[1], args[2]), 37, 500, 16)
+
+
+@pytest.mark.parametrize("cols", [33, 129, 4097, 131073, 1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("window", [3, 16])
+def test_split(spmm_npu, cols, window):
+    """Ratios that move nothing, everything, and part of an occupancy; a window
+    of more blocks than the LDS holds."""
+    crow, col = matrix(cols, seed=1)
+    args = as_types(crow, col, np.int32, np.float32)
+    for a in (0.0, 0.02, 295.0 / 505.0, 2.5, 40.0, 1e9, float("inf"), float("nan"), -1.0):
+        assert_same(spmm_npu.block_level_split(*gpu(*args), 37, cols, a, window),
+                    O.block_level_split(*args, 37, cols, a, window))
+
+
+def square(n, seed=0):
+    """Windows of different densities, a long row, occupancies from 1 to 16 and
+    a last window of n % 16 rows."""
+    rng = np.random.default_rng(n + seed)
+    parts = []
+    for r in range(n):
+        k = int(rng.integers(0, 6)) + (20 if (r // 16) % 5 == 0 else 0)
+        near = r // 16 * 16 + rng.integers(0, 48, k)
+        far = rng.integers(0, n, 3)
+        parts.append(np.unique(np.concatenate([near, far]) % n))
+    parts[min(40, n - 1)] = np.unique(rng.integers(0, n, min(n, 6000)))
+    crow = np.zeros(n + 1, np.int64)
+    crow[1:] = np.cumsum([p.size for p in parts])
+    return crow, np.concatenate(parts).astype(np.int64)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 100, 1600, 5003])
+@pytest.mark.parametrize("layout", [False, True])
+def test_preprocess(spmm_npu, n, layout):
+    crow, col = square(n)
+    for index, value in ((np.int32, np.float16), (np.int64, np.float32), (np.int32, np.float64)):
+        args = as_types(crow, col, index, value)
+        assert_same(spmm_npu.preprocess(*gpu(*args), n, n, graph_layout=layout),
+                    O.preprocess(*args, n, n, graph_layout=layout))
+
+
+@pytest.mark.parametrize("rows", [16 * 8192, 16 * 8192 + 5])
+def test_preprocess_either_side_of_the_window_sort(spmm_npu, rows):
+    """8192 windows are ranked by counting, more by the device sort."""
+    rng = np.random.default_rng(rows)
+    r = np.sort(rng.integers(0, rows, 40000))
+    key = np.unique(r * 3000 + rng.integers(0, 3000, r.size))
+    crow = np.zeros(rows + 1, np.int64)
+    crow[1:] = np.cumsum(np.bincount(key // 3000, minlength=rows))
+    args = as_types(crow, key % 3000, np.int32, np.float16)
+    assert_same(spmm_npu.preprocess(*gpu(*args), rows, 3000), O.preprocess(*args, rows, 3000))
+
+
+@pytest.mark.parametrize("cols", [4097, 300000, 1 << 20])
+def test_preprocess_wide_marginal_window(spmm_npu, cols):
+    """One window holds nearly all nonzeros, so it is the marginal one: its
+    blocks fit the LDS arrays, or not (2^20 columns leave no room)."""
+    crow, col = matrix(cols, seed=2)
+    args = as_types(crow, col, np.int32, np.float32)
+    assert_same(spmm_npu.preprocess(*gpu(*args), 37, cols), O.preprocess(*args, 37, cols))
+
+
+@pytest.mark.parametrize("n", [32768, 32769])
+def test_longest_window(spmm_npu, n):
+    """One nonzero more sends the matrix to the sorting pipeline."""
+    crow = np.array([0, n - 20000, n, n + 1], np.int64)
+    rng = np.random.default_rng(n)
+    col = np.concatenate([np.sort(rng.choice(40000, k, replace=False)) for k in (n - 20000, 20000, 1)])
+    crow, col = crow - np.array([0, 0, 1, 1]), np.delete(col, n - 1)  # n nonzeros in the one window
+    args = as_types(crow, col, np.int32, np.float16)
+    assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 3, 40000, 16), O.csr_to_bcsr(*args, 3, 40000, 16))
+    assert_same(spmm_npu.block_level_split(*gpu(*args), 3, 40000, 0.6, 16),
+                O.block_level_split(*args, 3, 40000, 0.6, 16))
+    assert_same(spmm_npu.preprocess(*gpu(*args), 3, 40000), O.preprocess(*args, 3, 40000))
+
+
+@pytest.mark.parametrize("layout", [False, True])
+def test_unsorted_rows_take_the_sorting_pipeline(spmm_npu, layout):
+    crow, col = square(333)
+    col = col.copy()
+    for r in range(0, 333, 7):
+        col[crow[r]:crow[r + 1]] = col[crow[r]:crow[r + 1]][::-1]
+    args = as_types(crow, col, np.int32, np.float32)
+    assert_same(spmm_npu.preprocess(*gpu(*args), 333, 333, graph_layout=layout),
+                O.preprocess(*args, 333, 333, graph_layout=layout))
+    assert_same(spmm_npu.block_level_split(*gpu(*args), 333, 333, 0.6, 16),
+                O.block_level_split(*args, 333, 333, 0.6, 16))
