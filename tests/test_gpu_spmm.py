@@ -397,6 +397,44 @@ def test_vector_path_width_invariant_bitwise(spmm_npu, dtype):
         assert torch.equal(part, full[:, :n]), f"width {n} differs"
 
 
+@pytest.mark.parametrize("dtype,width", [("fp16", 128), ("fp16", 256), ("fp16", 512), ("fp16", 1024),
+                                         ("fp32", 64), ("fp32", 128), ("fp32", 512)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_line_pieces_equal_narrow_rows_bitwise(spmm_npu, dtype, width, mixed):
+    """Rows of 8 to 64 nonzeros over a dense operand larger than one L2 take
+    column pieces of one cache line; C[:, :16], C[:, 16:32], ... computed alone
+    (dense rows too narrow for them) are the same bits.  Long rows cross ranges
+    and tiles, some columns are invalid, the row count is ragged, and in the
+    mixed operator one block window takes vector sums."""
+    rng = np.random.default_rng(311)
+    rows, cols = 16_411, 17_000
+    crow, col = random_csr(rng, rows, cols, 25, long_rows=[(5, 900), (8000, 3000), (rows - 1, 700)])
+    assert cols * 8 <= col.size <= rows * 64
+    col[[0, col.size // 2, col.size - 1]] = [cols, -1, cols + 7]
+    vals = rng.uniform(-1, 1, col.size).astype(NP_DT[dtype])
+    B = rng.standard_normal((cols, width)).astype(NP_DT[dtype])
+    assert B.nbytes > 4 << 20
+
+    def run(b):
+        if not mixed:
+            return run_csr(spmm_npu, crow, col, vals, b).cpu()
+        bvals = np.arange(32 * 16).reshape(-1) % 7 - 3.0
+        return spmm_npu.spmm_ascend_cube(
+            dev(np.array([0, 32], np.int32)), dev(np.arange(32, dtype=np.int32) * 500), dev(bvals.astype(NP_DT[dtype])),
+            dev(crow, torch.int32), dev(col, torch.int32), dev(vals), dev(b), zero_start(20),
+            dev(O.make_start(crow, 40))).cpu()
+
+    full = run(B)
+    step = 16 if width <= 256 else width // 4 - 16
+    for c in range(0, width, step):
+        part = run(np.ascontiguousarray(B[:, c:c + 16]))
+        assert torch.equal(part, full[:, c:c + 16]), f"columns {c} ff. differ"
+    if not mixed:
+        ok = (col >= 0) & (col < cols)
+        c2, v2 = np.where(ok, col, 0), np.where(ok, vals, 0).astype(NP_DT[dtype])
+        assert_close(full[:, :32], O.spmm_f64(crow, c2, v2, np.ascontiguousarray(B[:, :32])), dtype)
+
+
 @pytest.mark.parametrize("dtype,rows", [("fp16", 320), ("fp32", 320), ("fp16", 16 * 3000), ("fp32", 16 * 3000)])
 def test_block_path_width_invariant_bitwise(spmm_npu, dtype, rows):
     """Mixed operator on a preprocess layout (block part + vector part):
