@@ -154,13 +154,25 @@ size_t gather_workspace_bytes(int64_t nnz, int64_t width);
 // range costs a work-group and a window search), and growing with the total
 // block count (at most about 16384 chunks, 4096 blocks per chunk at most),
 // so large inputs keep the partial sums (and their workspace) small; it
-// depends on the value type and the block count only, never on the width,
+// depends on the value type, block and window counts only, never on the width,
 // so results do not depend on the width.  fp32 keeps 1024: the split also
 // bounds the fp32 accumulation chain of hub rows (config 5's rows of 8192
 // nonzeros miss the 1e-4 tolerance in 44 of 35M sampled elements with 4096).
-inline int64_t block_chunk_for(int32_t value_type, int64_t blocks) {
+//
+// Few windows leave the chip idle when a work-group sums up to 2048 blocks by
+// itself, so the fp16 chunk halves, to 512 at least, while windows and chunks
+// together are fewer than 4096 work-groups (256 CUs with 16 resident each).
+// The mixed operator on 2.0M power-law nonzeros (687 windows of 1070 blocks on
+// average), N = 128: 115 us with chunks of 2048, 111.6 with 1024, 108.4 with
+// 512; 256 lost it again (120.8: the partial sums).  fp32 stays at 1024: with
+// 512 a graph's training step (131072 rows of 30, N = 256), bound by the
+// fabric's rate already, went from 1443 to 1470 us.
+constexpr int64_t kBlockMinChunk = 512;
+constexpr int64_t kBlockWorkGroups = 4096;
+inline int64_t block_chunk_for(int32_t value_type, int64_t blocks, int64_t windows) {
   int64_t k = value_type == SPMM_VALUE_F16 ? 2048 : 1024;
   while (k < 4096 && blocks / k > 16384) k *= 2;
+  while (value_type == SPMM_VALUE_F16 && k > kBlockMinChunk && windows + blocks / k < kBlockWorkGroups) k /= 2;
   return k;
 }
 

@@ -1016,6 +1016,40 @@ def test_windows_longer_than_the_block_chunk(spmm_npu, dtype, width):
     assert_close(out[:rows], expected, dtype)
 
 
+@pytest.mark.parametrize("dtype,width", [("fp16", 64), ("fp16", 256), ("fp32", 64)])
+def test_windows_around_the_smallest_block_chunk(spmm_npu, dtype, width):
+    """Few windows take fp16 chunks of 512 blocks: windows of one block more
+    or less than one, two and three chunks, with a vector part (overflow
+    work-groups) and without (one work-group per window), against the oracle
+    and each other.  One nonzero per block."""
+    rng = np.random.default_rng(7 + width)
+    sizes = [511, 512, 513, 1, 1023, 1024, 1025, 0, 1535, 1537]
+    rows, K = 16 * len(sizes), 4000
+    parts = [[] for _ in range(rows)]
+    for s, n in enumerate(sizes):
+        for k, c in enumerate(np.sort(rng.choice(K, n, replace=False))):
+            parts[16 * s + k % 16].append(c)
+    crow = np.zeros(rows + 1, np.int64)
+    crow[1:] = np.cumsum([len(p) for p in parts])
+    col = np.concatenate([np.asarray(p, np.int64) for p in parts])
+    vals = rng.uniform(-1, 1, col.size).astype(NP_DT[dtype])
+    B = rng.standard_normal((K, width)).astype(NP_DT[dtype])
+    i32 = torch.int32
+    b = O.csr_to_bcsr(crow, col, vals, rows, K, 16)
+    assert np.diff(b["crow_window_ptr"]).tolist() == sizes
+    bops = (dev(b["crow_window_ptr"], i32), dev(b["unique_col_ids"], i32), dev(b["value"]))
+    bstart = dev(O.make_start(b["crow_window_ptr"], 20))
+    out = spmm_npu.spmm_ascend_cube(*bops, zero_start(1), torch.zeros(0, dtype=i32, device="cuda"),
+                                    torch.zeros(0, dtype=dev(vals).dtype, device="cuda"), dev(B), bstart,
+                                    zero_start(40))
+    assert_close(out[:rows], O.spmm_f64(crow, col, vals, B), dtype)
+    vrow = np.ones(rows + 1, np.int64)
+    vrow[0] = 0
+    out_v = spmm_npu.spmm_ascend_cube(*bops, dev(vrow, i32), torch.zeros(1, dtype=i32, device="cuda"),
+                                      dev(np.ones(1, NP_DT[dtype])), dev(B), bstart, dev(O.make_start(vrow, 40)))
+    assert torch.equal(out_v[1:rows], out[1:rows])
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "fp16"])
 def test_column_passes_equal_single_pass_bitwise(spmm_npu, dtype):
     """A dense operand of more than 512 MiB (K = 600k rows: fp32 N = 512, or
