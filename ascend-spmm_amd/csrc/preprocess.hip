@@ -1572,7 +1572,7 @@ spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
     if (spmm_status st = win::plan_task(wm, layout, B.x, s)) return st;
     win::TaskRecord v;
     if (spmm_status st = read_back(&v, B.x.record, 1, s)) return st;
-    if (v.err == 0) {
+    if (v.err == 0 && v.t_err == 0) {
       spmm_taskmap_info r{};
       r.aic_windows = v.naic;
       r.aic_blocks = v.aic_blocks;

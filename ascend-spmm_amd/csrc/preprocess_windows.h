@@ -58,6 +58,7 @@ struct TaskRecord {
   int64_t out_rows;
   double est_aic, est_aiv, est_max;
   int64_t t_kept, t_vnnz;  // graph layout: the transpose's split
+  int64_t t_err;           // its error word (err is read, so not written, by its kernels)
 };
 
 // block_level_split, and the graph layout's transpose.

@@ -1226,17 +1226,23 @@ __device__ inline void count_occupancy(const Cols& cols_at, const RowStarts& s, 
 }
 
 // Blocks per window by occupancy, and their sums over all windows (spread over
-// kHistCopies counters: same-address atomics run one after another).
-template <typename P, typename Cols, bool kCheck, typename State>
+// kHistCopies counters: same-address atomics run one after another).  `stop`
+// (or null) is an error word of earlier kernels, which makes this one leave;
+// it stores its own errors to `err`, a different word: were it the same one,
+// the wavefronts of a work-group could read it before and after another
+// work-group's store, and those that stayed would use the LDS of those that
+// left, and write by it.
+template <typename P, typename Cols, bool kCheck>
 __global__ __launch_bounds__(1024) void split_counts(const P* __restrict__ rowptr, Cols col, int64_t rows,
                                                      int64_t cols, int64_t nnz, int W, uint32_t words, uint32_t groups,
                                                      int gshift, uint32_t* __restrict__ nb, uint32_t* __restrict__ hist,
-                                                     uint32_t* __restrict__ total, uint32_t* occ_far, State* st) {
+                                                     uint32_t* __restrict__ total, uint32_t* occ_far,
+                                                     const int64_t* stop, int64_t* err) {
   extern __shared__ __align__(16) uint32_t bm[];
   uint32_t* const prefix = bm + words;
   __shared__ WindowRows s;
   __shared__ uint32_t s_wave[17], s_hist[32];
-  if (!kCheck && st->err != 0) return;
+  if (stop != nullptr && *stop != 0) return;  // uniform: not written in this launch
   const int64_t w = blockIdx.x;
   clear_words(bm, words);
   if (threadIdx.x < 32) s_hist[threadIdx.x] = 0u;
@@ -1245,7 +1251,7 @@ __global__ __launch_bounds__(1024) void split_counts(const P* __restrict__ rowpt
   int bad = s.ok && !long_window(s.n, nnz) ? 0 : 1;
   const RowStarts starts(s);
   if (!bad) set_bits<kCheck>(col, starts, cols, bm, held, &bad);  // uniform
-  if (bad) st->err = kGeneral;
+  if (bad) *err = kGeneral;
   if (__syncthreads_or(bad)) return;
   const uint32_t blocks = bitmap_prefix(bm, prefix, words, gshift, s_wave);
   const bool near = blocks <= kOccLds;
@@ -1293,20 +1299,20 @@ struct SplitCost {
 // after it: the minimum is at that k or before it, and binary searches find
 // its first place.  Then, per window, its share of the boundary occupancy's
 // blocks, and prefix sums of kept blocks and moved nonzeros.  One work-group.
-template <typename State>
+// stop, err: as for split_counts, written by earlier kernels only.
 __global__ __launch_bounds__(1024) void split_decide(int64_t nwin, double a,
                                                      const uint32_t* __restrict__ nb,
                                                      const uint32_t* __restrict__ hist,
                                                      const uint32_t* __restrict__ total, uint32_t* __restrict__ moved,
                                                      uint32_t* __restrict__ kptr, uint32_t* __restrict__ vptr,
-                                                     uint32_t* __restrict__ rule, State* st, int64_t* kept_out,
-                                                     int64_t* vnnz_out) {
+                                                     uint32_t* __restrict__ rule, const int64_t* stop,
+                                                     const int64_t* err, int64_t* kept_out, int64_t* vnnz_out) {
   __shared__ SplitCost f;
   __shared__ uint32_t s_wave[17], s_h[16], s_edge;
   __shared__ uint64_t s_wave64[17];
   __shared__ int64_t s_k;
   const uint32_t tid = threadIdx.x;
-  if (st->err != 0) return;
+  if (*err != 0 || (stop != nullptr && *stop != 0)) return;
   if (tid < 16) s_h[tid] = 0u;
   __syncthreads();
   for (uint32_t t = tid; t < 16 * kHistCopies; t += 1024) {
@@ -1600,16 +1606,18 @@ spmm_status fill_blocks(const Matrix& m, int64_t W, bool tiles, const BlockArray
 
 namespace {
 
-template <typename P, typename Cols, bool kCheck, typename State>
+template <typename P, typename Cols, bool kCheck>
 spmm_status run_split(const P* rowptr, Cols col, int64_t rows, int64_t cols, int64_t nnz, double a, int64_t W,
-                      const SplitArrays& x, State* st, int64_t* kept, int64_t* vnnz, hipStream_t s) {
+                      const SplitArrays& x, const int64_t* stop, int64_t* err, int64_t* kept, int64_t* vnnz,
+                      hipStream_t s) {
   const int64_t nwin = ceil_div(rows, W);
   const BitmapShape b(cols, nnz, nwin);
   const size_t lds = b.lds() + kOccLds * sizeof(uint32_t);
-  hipLaunchKernelGGL((split_counts<P, Cols, kCheck, State>), dim3(static_cast<unsigned>(nwin)), dim3(b.threads(lds)), lds, s, rowptr, col, rows, cols, nnz, static_cast<int>(W),
-                     b.words, b.groups, b.gshift, x.nb, x.hist, x.total, x.occ, st);
-  hipLaunchKernelGGL(split_decide<State>, dim3(1), dim3(1024), 0, s, nwin, a, x.nb, x.hist, x.total,
-                     x.moved, x.kptr, x.vptr, x.rule, st, kept, vnnz);
+  hipLaunchKernelGGL((split_counts<P, Cols, kCheck>), dim3(static_cast<unsigned>(nwin)), dim3(b.threads(lds)), lds, s,
+                     rowptr, col, rows, cols, nnz, static_cast<int>(W), b.words, b.groups, b.gshift, x.nb, x.hist,
+                     x.total, x.occ, stop, err);
+  hipLaunchKernelGGL(split_decide, dim3(1), dim3(1024), 0, s, nwin, a, x.nb, x.hist, x.total, x.moved, x.kptr, x.vptr,
+                     x.rule, stop, static_cast<const int64_t*>(err), kept, vnnz);
   return check_launch("split counts");
 }
 
@@ -1632,9 +1640,9 @@ spmm_status plan_split(const Matrix& m, double a, int64_t W, const SplitArrays& 
   return by_index(m.index_type, [&](auto i) {
     using I = decltype(i);
     init_state(state, x.total, 16 * kHistCopies, s);
-    return run_split<I, CsrColumns<I>, true, WindowState>(static_cast<const I*>(m.rowptr),
-                                                          CsrColumns<I>{static_cast<const I*>(m.col)}, m.rows, m.cols,
-                                                          m.nnz, a, W, x, state, &state->total, &state->vnnz, s);
+    return run_split<I, CsrColumns<I>, true>(static_cast<const I*>(m.rowptr),
+                                             CsrColumns<I>{static_cast<const I*>(m.col)}, m.rows, m.cols, m.nnz, a, W,
+                                             x, nullptr, &state->err, &state->total, &state->vnnz, s);
   });
 }
 
@@ -1726,9 +1734,9 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, hipStre
       return check_hip(e, "transpose sort");
     hipLaunchKernelGGL(transpose_starts, dim3(static_cast<unsigned>(ceil_div(m.nnz + 1, 256))), dim3(256), 0, s,
                        x.stkey, m.nnz, 16 * nwin, x.record, x.rp);
-    return run_split<uint32_t, WordColumns, false, TaskRecord>(x.rp, WordColumns{x.stword}, 16 * nwin, 16 * nwin,
-                                                               m.nnz, 295.0 / 505.0, 16, x.split, x.record,
-                                                               &x.record->t_kept, &x.record->t_vnnz, s);
+    return run_split<uint32_t, WordColumns, false>(x.rp, WordColumns{x.stword}, 16 * nwin, 16 * nwin, m.nnz,
+                                                   295.0 / 505.0, 16, x.split, &x.record->err, &x.record->t_err,
+                                                   &x.record->t_kept, &x.record->t_vnnz, s);
   });
 }
 

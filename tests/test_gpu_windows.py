@@ -178,6 +178,28 @@ def test_longest_window(spmm_npu, n):
     assert_same(spmm_npu.preprocess(*gpu(*args), 3, 40000), O.preprocess(*args, 3, 40000))
 
 
+def hub_column(n, hub, seed=4):
+    """Short rows, the first `hub` of which hold column 7 too."""
+    rng = np.random.default_rng(seed)
+    key = np.unique(np.concatenate([np.arange(hub) * n + 7, rng.integers(0, n, 2 * n) + np.arange(2 * n) // 2 * n]))
+    crow = np.zeros(n + 1, np.int64)
+    crow[1:] = np.cumsum(np.bincount(key // n, minlength=n))
+    return crow, key % n
+
+
+@pytest.mark.parametrize("hub", [32000, 40000])
+def test_hub_column_of_the_packed_transpose(spmm_npu, hub):
+    """No window of A is long, but the transpose's window that holds the hub
+    column is: of at most 32768 nonzeros (taken window by window), or more
+    (only the transpose's split finds that out, after its other windows have
+    begun, and the matrix goes to the sorting pipeline)."""
+    n = 40000
+    crow, col = hub_column(n, hub)
+    assert np.diff(crow[::16]).max() < 64
+    args = as_types(crow, col, np.int32, np.float32)
+    assert_same(spmm_npu.preprocess(*gpu(*args), n, n, graph_layout=True), O.preprocess(*args, n, n, graph_layout=True))
+
+
 @pytest.mark.parametrize("layout", [False, True])
 def test_unsorted_rows_take_the_sorting_pipeline(spmm_npu, layout):
     crow, col = square(333)
