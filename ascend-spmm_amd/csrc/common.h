@@ -154,25 +154,22 @@ size_t gather_workspace_bytes(int64_t nnz, int64_t width);
 // range costs a work-group and a window search), and growing with the total
 // block count (at most about 16384 chunks, 4096 blocks per chunk at most),
 // so large inputs keep the partial sums (and their workspace) small; it
-// depends on the value type, block and window counts only, never on the width,
+// depends on the value type and the block count only, never on the width,
 // so results do not depend on the width.  fp32 keeps 1024: the split also
 // bounds the fp32 accumulation chain of hub rows (config 5's rows of 8192
 // nonzeros miss the 1e-4 tolerance in 44 of 35M sampled elements with 4096).
 //
-// Few windows leave the chip idle when a work-group sums up to 2048 blocks by
-// itself, so the fp16 chunk halves, to 512 at least, while windows and chunks
-// together are fewer than 4096 work-groups (256 CUs with 16 resident each).
-// The mixed operator on 2.0M power-law nonzeros (687 windows of 1070 blocks on
-// average), N = 128: 115 us with chunks of 2048, 111.6 with 1024, 108.4 with
-// 512; 256 lost it again (120.8: the partial sums).  fp32 stays at 1024: with
-// 512 a graph's training step (131072 rows of 30, N = 256), bound by the
-// fabric's rate already, went from 1443 to 1470 us.
-constexpr int64_t kBlockMinChunk = 512;
-constexpr int64_t kBlockWorkGroups = 4096;
-inline int64_t block_chunk_for(int32_t value_type, int64_t blocks, int64_t windows) {
+// Few long windows leave the chip idle, but smaller fp16 chunks for them lose
+// more than they gain, as a piece costs its stores and reads at the device
+// coherence point and takes the kernel's 4-column path: with 512, 1024 windows
+// of 600 / 1100 blocks without a vector part take 26.1 -> 52.5 / 34.0 -> 78.5
+// us at N = 256, 256 windows of 600 14.7 -> 19.7 at N = 128; in the mixed
+// operator 540 windows of 2000 blocks 140 -> 206 us at N = 256 and 96 -> 105
+// at N = 128, where 687 power-law windows of 1070 on average gain 115 -> 108.
+// Sizes do not tell these apart, and the chunk must not depend on the width.
+inline int64_t block_chunk_for(int32_t value_type, int64_t blocks) {
   int64_t k = value_type == SPMM_VALUE_F16 ? 2048 : 1024;
   while (k < 4096 && blocks / k > 16384) k *= 2;
-  while (value_type == SPMM_VALUE_F16 && k > kBlockMinChunk && windows + blocks / k < kBlockWorkGroups) k /= 2;
   return k;
 }
 

@@ -32,7 +32,7 @@
 //  * Waves of the work-group take column groups round-robin; each group
 //    runs the whole K loop, so every output element sees the same MFMA
 //    sequence for every width N.
-//  * Windows longer than a chunk (block_chunk_for: 512-2048 blocks fp16, 1024
+//  * Windows longer than a chunk (block_chunk_for: 2048 blocks fp16, 1024
 //    fp32, growing with the total block count) are cut at fixed block
 //    positions: the window's own work-group takes its first chunk, and
 //    "overflow" work-groups take the rest in fixed global block ranges (only
@@ -703,7 +703,7 @@ spmm_status block_typed(const void* Crowptr, const void* Ccol, const void* Cvalu
   a.zero_empty = vector_nnz == 0 ? 1 : 0;
   a.order = order;
   a.serial = counters_zeroed ? 0 : 1;
-  a.kbig = block_chunk_for(sizeof(T) == 2 ? SPMM_VALUE_F16 : SPMM_VALUE_F32, a.limit, windows);
+  a.kbig = block_chunk_for(sizeof(T) == 2 ? SPMM_VALUE_F16 : SPMM_VALUE_F32, a.limit);
   a.noverflow = block_overflow_ranges(a.limit, a.kbig);
   a.cnt = reinterpret_cast<uint32_t*>(slots + a.noverflow * 2 * 16 * N);
   a.per_xcd = ceil_div(windows, kXcds * kBlockXcdRun) * kBlockXcdRun;

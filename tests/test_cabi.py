@@ -94,6 +94,25 @@ def test_host_validation_without_gpu(lib):
     assert b"more than the library's fixed" in lib.spmm_last_error()
 
 
+@pytest.mark.parametrize("windows", [1, 64, 687, 3000])
+@pytest.mark.parametrize("vector_nnz", [0, 5000])
+def test_fp16_windows_of_up_to_2048_blocks_leave_no_pieces(lib, windows, vector_nnz):
+    """The partial sums of windows longer than the block chunk take workspace;
+    the chunk is 2048 blocks for fp16 however few the windows are (smaller
+    ones cost such calls up to twice the time)."""
+    def bytes_for(blocks):
+        m = MixedDesc(windows, blocks, 16 * blocks, 16 * windows, vector_nnz, 4000, 128, 0, 0)
+        size = ctypes.c_size_t(0)
+        assert lib.spmm_mixed_workspace(ctypes.byref(m), ctypes.byref(size)) == 0
+        return size.value
+
+    assert bytes_for(2048) == bytes_for(1)
+    # past it: one range per 2048 blocks, two 16 x 128 fp32 pieces and a counter each
+    for blocks, ranges in ((2049, 2), (4096, 2), (4097, 3), (700_000, 342)):
+        pieces = ranges * (2 * 16 * 128 * 4 + 4)
+        assert bytes_for(blocks) - bytes_for(1) == -(-pieces // 256) * 256
+
+
 @pytest.mark.gpu
 def test_direct_cabi_calls_match_oracle(lib):
     import torch

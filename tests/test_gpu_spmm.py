@@ -1017,14 +1017,15 @@ def test_windows_longer_than_the_block_chunk(spmm_npu, dtype, width):
 
 
 @pytest.mark.parametrize("dtype,width", [("fp16", 64), ("fp16", 256), ("fp32", 64)])
-def test_windows_around_the_smallest_block_chunk(spmm_npu, dtype, width):
-    """Few windows take fp16 chunks of 512 blocks: windows of one block more
-    or less than one, two and three chunks, with a vector part (overflow
-    work-groups) and without (one work-group per window), against the oracle
-    and each other.  One nonzero per block."""
+def test_windows_around_the_block_chunk(spmm_npu, dtype, width):
+    """Windows of one block more or less than one, two and three chunks (2048
+    blocks fp16, 1024 fp32), with a vector part (overflow work-groups) and
+    without (one work-group per window), against the oracle and each other.
+    One nonzero per block."""
     rng = np.random.default_rng(7 + width)
-    sizes = [511, 512, 513, 1, 1023, 1024, 1025, 0, 1535, 1537]
-    rows, K = 16 * len(sizes), 4000
+    chunk = {"fp16": 2048, "fp32": 1024}[dtype]
+    sizes = [chunk - 1, chunk, chunk + 1, 1, 2 * chunk - 1, 2 * chunk, 2 * chunk + 1, 0, 3 * chunk - 1, 3 * chunk + 1]
+    rows, K = 16 * len(sizes), 8000
     parts = [[] for _ in range(rows)]
     for s, n in enumerate(sizes):
         for k, c in enumerate(np.sort(rng.choice(K, n, replace=False))):
