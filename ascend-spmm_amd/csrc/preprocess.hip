@@ -1234,7 +1234,7 @@ template <typename I>
 spmm_status bcsr_plan(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStream_t s,
                       bool tiles, int64_t* count, spmm_plan_record* record) {
   const win::Matrix wm = window_matrix(c);
-  if (win::eligible(wm, W)) {
+  if (win::eligible(win::Op::kBlocks, wm, W)) {
     const WindowBlocks B(c, W, ws);
     if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
     if (spmm_status st = win::plan_blocks(wm, W, tiles, B.a, s)) return st;
@@ -1425,7 +1425,7 @@ template <typename I>
 spmm_status hybrid_plan(const Csr& c, double a, int64_t W, void* ws, size_t ws_bytes, hipStream_t s,
                         int64_t* kept, int64_t* vnnz, spmm_plan_record* record) {
   const win::Matrix wm = window_matrix(c);
-  if (win::eligible(wm, W)) {
+  if (win::eligible(win::Op::kSplit, wm, W)) {
     const WindowSplit B(c, W, ws);
     if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
     if (spmm_status st = win::plan_split(wm, a, W, B.x, B.state, s)) return st;
@@ -1550,11 +1550,8 @@ void lay_task(Ctx& x, TaskArrays& A, const Csr& c, bool layout, void* ws) {
   A.lay(x.arena, c, layout);
 }
 
-// The window-by-window pipeline takes the matrix, and its transpose's columns
-// (packed rows) too where the graph layout asks for it.
 bool window_task_eligible(const Csr& c, bool graph_layout) {
-  return win::eligible(window_matrix(c), 16) &&
-         (!(graph_layout && c.rows == c.cols) || 16 * ceil_div(c.rows, 16) <= win::kMaxColumns);
+  return win::eligible(graph_layout && c.rows == c.cols ? win::Op::kTaskLayout : win::Op::kTask, window_matrix(c), 16);
 }
 
 Csr transposed_csr(const Csr& c, const TaskArrays& A, int64_t out_rows, int64_t n) {
@@ -1819,7 +1816,9 @@ size_t bcsr_bytes(const spmm_csr_matrix* m, int64_t W, bool tiles) {
   CubeExtra cube;
   const Csr c = from_matrix(m);
   lay_bcsr(x, S, tiles ? &cube : nullptr, c, W, nullptr);
-  return win::eligible(window_matrix(c), W) ? std::max(x.arena.used, WindowBlocks(c, W, nullptr).used) : x.arena.used;
+  return win::eligible(win::Op::kBlocks, window_matrix(c), W)
+             ? std::max(x.arena.used, WindowBlocks(c, W, nullptr).used)
+             : x.arena.used;
 }
 
 }  // namespace
@@ -1929,7 +1928,9 @@ size_t spmm_hybrid_workspace(const spmm_csr_matrix* m, int64_t W) {
   HybridArrays H;
   const Csr c = from_matrix(m);
   lay_hybrid(x, H, c, W, nullptr);
-  return win::eligible(window_matrix(c), W) ? std::max(x.arena.used, WindowSplit(c, W, nullptr).used) : x.arena.used;
+  return win::eligible(win::Op::kSplit, window_matrix(c), W)
+             ? std::max(x.arena.used, WindowSplit(c, W, nullptr).used)
+             : x.arena.used;
 }
 
 static spmm_status split_plan(const spmm_csr_matrix* m, double a, int64_t W, void* ws, size_t ws_bytes, spmm_stream s,

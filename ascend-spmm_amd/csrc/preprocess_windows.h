@@ -1,21 +1,17 @@
 // Window-by-window preprocessing (preprocess_windows.hip): host interface used
 // by the pipelines of preprocess.hip.
 //
-// Applies to matrices whose rows hold strictly ascending column ids, with at
-// most kMaxColumns columns, fewer than 2^31 nonzeros and windows of at most 16
-// rows (eligible() checks the sizes; the plan kernels check the rest and set
-// WindowState::err otherwise, and the caller then takes the sorting pipeline,
-// which also reports every input error).
+// Applies to matrices whose rows hold strictly ascending column ids, of the
+// sizes that window_rule.h takes (the plan kernels check the rest and set the
+// record's error word otherwise, and the caller then takes the sorting
+// pipeline, which also reports every input error).
 #pragma once
 
 #include "common.h"
+#include "window_rule.h"
 
 namespace spmm {
 namespace win {
-
-// A window's column set is a bitmap in LDS, one bit per column: 2^20 columns
-// are 128 KB, beside 16 KB of prefix counts.
-constexpr int64_t kMaxColumns = int64_t(1) << 20;
 
 struct Matrix {
   int64_t rows, cols, nnz;
@@ -25,10 +21,7 @@ struct Matrix {
   const void* value;
 };
 
-inline bool eligible(const Matrix& m, int64_t W) {
-  return W >= 1 && W <= 16 && m.rows >= 1 && m.cols >= 1 && m.cols <= kMaxColumns && m.nnz >= 1 &&
-         m.nnz < (int64_t(1) << 31) && m.rows < (int64_t(1) << 31) - 64;
-}
+inline bool eligible(Op op, const Matrix& m, int64_t W) { return eligible(op, m.rows, m.cols, m.nnz, W); }
 
 // Device record of a plan, read back by the host in one copy.
 struct WindowState {

@@ -1,0 +1,45 @@
+"""Which conversions go window by window (ascend-spmm_amd/csrc/window_rule.h):
+the rule is host arithmetic on the sizes, compiled here by itself."""
+
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ascend-spmm_amd", "csrc")
+BLOCKS, SPLIT, TASK, TASK_LAYOUT = range(4)
+
+
+@pytest.fixture(scope="module")
+def eligible(tmp_path_factory):
+    out = tmp_path_factory.mktemp("rule")
+    source, library = out / "rule.cpp", out / "rule.so"
+    source.write_text('#include "window_rule.h"\n'
+                      'extern "C" int rule(int op, long long rows, long long cols, long long nnz, long long w) {\n'
+                      "  return spmm::win::eligible(static_cast<spmm::win::Op>(op), rows, cols, nnz, w);\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", CSRC, str(source), "-o", str(library)],
+                   check=True)
+    rule = ctypes.CDLL(str(library)).rule
+    rule.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
+    return lambda *a: bool(rule(*a))
+
+
+@pytest.mark.parametrize("op", [BLOCKS, SPLIT, TASK])
+@pytest.mark.parametrize("window", [1, 3, 16])
+def test_windows_fit_a_grid_of_1024_threads_each(eligible, op, window):
+    """A grid of one work-group per window stays below 2^32 threads."""
+    most = 2**32 // 1024 - 1
+    nnz = 2**31 - 1
+    assert eligible(op, window * most, 64, nnz, window)
+    assert not eligible(op, window * most + 1, 64, nnz, window)
+    assert not eligible(op, 2**31 - 100, 64, nnz, window)
+
+
+def test_sizes_the_kernels_do_not_hold(eligible):
+    assert eligible(BLOCKS, 4096, 2**20, 10**6, 16) and not eligible(BLOCKS, 4096, 2**20 + 1, 10**6, 16)
+    assert not eligible(BLOCKS, 4096, 4096, 2**31, 16)
+    for rows, cols, nnz, window in ((0, 5, 5, 16), (5, 0, 5, 16), (5, 5, 0, 16), (5, 5, 5, 0), (5, 5, 5, 17)):
+        assert not eligible(SPLIT, rows, cols, nnz, window)
+    # the transpose's columns are the packed rows, whole windows of them
+    assert eligible(TASK_LAYOUT, 2**20, 2**20, 2**28, 16) and not eligible(TASK_LAYOUT, 2**20 + 1, 2**20, 2**28, 16)
