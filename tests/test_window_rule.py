@@ -43,3 +43,36 @@ def test_sizes_the_kernels_do_not_hold(eligible):
         assert not eligible(SPLIT, rows, cols, nnz, window)
     # the transpose's columns are the packed rows, whole windows of them
     assert eligible(TASK_LAYOUT, 2**20, 2**20, 2**28, 16) and not eligible(TASK_LAYOUT, 2**20 + 1, 2**20, 2**28, 16)
+
+
+K20 = 2**20
+# (op, rows, columns, nonzeros, window), the sorting and the window pipeline's
+# times on them (us): more columns, rows, nonzeros or smaller windows decide.
+MEASURED = [
+    (BLOCKS, K20, K20, 1 << 20, 16, 381, 3065), (BLOCKS, K20, K20, 1 << 20, 1, 365, 48000),
+    (BLOCKS, K20, K20, 1 << 24, 16, 2289, 3225), (BLOCKS, 1 << 18, 1 << 18, 1 << 20, 16, 370, 206),
+    (BLOCKS, K20, 1 << 12, 1 << 22, 16, 647, 441), (BLOCKS, K20, 1 << 12, 1 << 18, 16, 264, 417),
+    (BLOCKS, 1 << 16, 1 << 12, 1 << 19, 1, 288, 412), (BLOCKS, 1 << 12, K20, 1 << 18, 16, 281, 43),
+    (SPLIT, K20, K20, 1 << 20, 1, 672, 41668), (SPLIT, K20, 1 << 19, 1 << 22, 16, 1280, 1366),
+    (SPLIT, 1 << 15, K20, 1 << 15, 16, 350, 120), (SPLIT, K20, 1 << 12, 1 << 20, 4, 676, 1390),
+    (TASK, K20, K20, 1 << 22, 16, 1280, 2011), (TASK, 1 << 19, 1 << 19, 1 << 23, 16, 1816, 588),
+    (TASK, K20, 1 << 18, 1 << 18, 16, 685, 716), (TASK, 1 << 18, 1 << 18, 1 << 20, 16, 745, 269),
+    (TASK_LAYOUT, K20, K20, 1 << 22, 16, 2984, 5030), (TASK_LAYOUT, 1 << 18, 1 << 18, 1 << 22, 16, 2776, 724),
+]
+
+
+@pytest.mark.parametrize("op,rows,cols,nnz,window,sorting,windows", MEASURED)
+def test_the_faster_pipeline_is_tried(eligible, op, rows, cols, nnz, window, sorting, windows):
+    assert eligible(op, rows, cols, nnz, window) == (windows < sorting)
+
+
+@pytest.mark.parametrize("op", [BLOCKS, SPLIT, TASK, TASK_LAYOUT])
+def test_more_windows_or_columns_never_turn_a_matrix_eligible(eligible, op):
+    """One change from eligible to not along rows (at fixed nonzeros) and columns."""
+    def changes(flags):
+        assert flags[0] and not flags[-1]
+        return sum(a != b for a, b in zip(flags, flags[1:]))
+
+    rows = [1 << k for k in range(4, 21)]
+    assert changes([eligible(op, r, 1 << 12, 1 << 16, 1) for r in rows]) == 1
+    assert changes([eligible(op, 1 << 18, 1 << k, 1 << 18, 16) for k in range(8, 21)]) == 1
