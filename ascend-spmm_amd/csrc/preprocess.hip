@@ -1050,22 +1050,39 @@ spmm_status zero(void* p, int64_t bytes, hipStream_t s) {
   return check_launch("zero fill");
 }
 
+// First position and nonzeros of a matrix whose row pointer has been found
+// monotone inside [0, nnz] already; n < 0: not known.
+struct Ends {
+  int64_t p_begin = 0, n = -1;
+};
+
+// Of a window plan that handed its matrix over (its record has been read back).
+template <typename Record>
+Ends ends_of(const Record& v) {
+  return win::ends_known(v.err) ? Ends{v.p_begin, v.n} : Ends{};
+}
+
 template <typename I>
-spmm_status run_window_sort(const Csr& c, int64_t W, bool check_sorted, WinSort& S, Ctx& x) {
+spmm_status run_window_sort(const Csr& c, int64_t W, bool check_sorted, const Ends& ends, WinSort& S, Ctx& x) {
   hipStream_t s = x.stream;
   launch(fill_kernel<int>, 4, s, S.err, int64_t(4), 0);
-  if (c.rows > 0)
-    launch(check_rowptr<I>, c.rows, s, static_cast<const I*>(c.rowptr), c.rows, c.nnz, S.err);
-  if (spmm_status st = check_launch("check_rowptr")) return st;
-  hipLaunchKernelGGL(collect_ends<I>, dim3(1), dim3(64), 0, s, static_cast<const I*>(c.rowptr), c.rows, S.err,
-                     S.scal);
-  int64_t v[3] = {0, 0, 0};
-  if (spmm_status st = read_back(v, S.scal, 3, s)) return st;
-  if (v[2] & kBadRowptr)
-    return fail(SPMM_ERR_INVALID_ARGUMENT,
-                "invalid CSR row pointer: entries must be non-decreasing within [0, nnz]");
-  S.p_begin = v[0];
-  S.n = v[1] - S.p_begin;
+  if (ends.n >= 0) {
+    S.p_begin = ends.p_begin;
+    S.n = ends.n;
+  } else {
+    if (c.rows > 0)
+      launch(check_rowptr<I>, c.rows, s, static_cast<const I*>(c.rowptr), c.rows, c.nnz, S.err);
+    if (spmm_status st = check_launch("check_rowptr")) return st;
+    hipLaunchKernelGGL(collect_ends<I>, dim3(1), dim3(64), 0, s, static_cast<const I*>(c.rowptr), c.rows, S.err,
+                       S.scal);
+    int64_t v[3] = {0, 0, 0};
+    if (spmm_status st = read_back(v, S.scal, 3, s)) return st;
+    if (v[2] & kBadRowptr)
+      return fail(SPMM_ERR_INVALID_ARGUMENT,
+                  "invalid CSR row pointer: entries must be non-decreasing within [0, nnz]");
+    S.p_begin = v[0];
+    S.n = v[1] - S.p_begin;
+  }
 
   if (c.rows > 0 && S.n > 0)
     launch(expand_rows<I>, (S.n + kExpandChunk - 1) / kExpandChunk * kT, s,
@@ -1233,6 +1250,7 @@ spmm_status load_header(Header& h, const Header* device, const spmm_plan_record*
 template <typename I>
 spmm_status bcsr_plan(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStream_t s,
                       bool tiles, int64_t* count, spmm_plan_record* record) {
+  Ends ends;
   const win::Matrix wm = window_matrix(c);
   if (win::eligible(win::Op::kBlocks, wm, W)) {
     const WindowBlocks B(c, W, ws);
@@ -1244,6 +1262,7 @@ spmm_status bcsr_plan(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStr
       *count = v.total;
       return store_header(Header{kMagicWindows, v.p_begin, v.n, v.total, 0, 0, 0, 0}, B.header, record, s);
     }
+    ends = ends_of(v);
   }
   Ctx x;
   WinSort S;
@@ -1252,7 +1271,7 @@ spmm_status bcsr_plan(const Csr& c, int64_t W, void* ws, size_t ws_bytes, hipStr
   x.prims.stream = s;
   lay_bcsr(x, S, tiles ? &cube : nullptr, c, W, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
-  if (spmm_status st = run_window_sort<I>(c, W, true, S, x)) return st;
+  if (spmm_status st = run_window_sort<I>(c, W, true, ends, S, x)) return st;
   Header h{kMagic, S.p_begin, S.n, S.nb, 0, 0, 0, 0};
   if (tiles) {
     launch(tile_counts, S.nwin + 1, s, S.win_start, S.nwin, cube.tiles);
@@ -1346,11 +1365,11 @@ struct HybridArrays {
 
 // Runs hybrid_split_impl up to the output sizes (kept blocks, vector nnz).
 template <typename I>
-spmm_status hybrid_run(const Csr& c, double a, int64_t W, HybridArrays& H, Ctx& x, int64_t* kept_out,
-                       int64_t* vnnz_out) {
+spmm_status hybrid_run(const Csr& c, double a, int64_t W, const Ends& ends, HybridArrays& H, Ctx& x,
+                       int64_t* kept_out, int64_t* vnnz_out) {
   hipStream_t s = x.stream;
   WinSort& S = H.S;
-  if (spmm_status st = run_window_sort<I>(c, W, false, S, x)) return st;
+  if (spmm_status st = run_window_sort<I>(c, W, false, ends, S, x)) return st;
   const int64_t nb = S.nb;
   // Block order: one sort on split_keys (occupancy, then first element),
   // unless an occupancy needs more than cbits; then (second round) the
@@ -1424,6 +1443,7 @@ void lay_hybrid(Ctx& x, HybridArrays& H, const Csr& c, int64_t W, void* ws) {
 template <typename I>
 spmm_status hybrid_plan(const Csr& c, double a, int64_t W, void* ws, size_t ws_bytes, hipStream_t s,
                         int64_t* kept, int64_t* vnnz, spmm_plan_record* record) {
+  Ends ends;
   const win::Matrix wm = window_matrix(c);
   if (win::eligible(win::Op::kSplit, wm, W)) {
     const WindowSplit B(c, W, ws);
@@ -1436,6 +1456,7 @@ spmm_status hybrid_plan(const Csr& c, double a, int64_t W, void* ws, size_t ws_b
       *vnnz = v.vnnz;
       return store_header(Header{kMagicWindows, 0, 0, 0, v.total, v.vnnz, 0, 0}, B.header, record, s);
     }
+    ends = ends_of(v);
   }
   Ctx x;
   HybridArrays H;
@@ -1443,7 +1464,7 @@ spmm_status hybrid_plan(const Csr& c, double a, int64_t W, void* ws, size_t ws_b
   x.prims.stream = s;
   lay_hybrid(x, H, c, W, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
-  if (spmm_status st = hybrid_run<I>(c, a, W, H, x, kept, vnnz)) return st;
+  if (spmm_status st = hybrid_run<I>(c, a, W, ends, H, x, kept, vnnz)) return st;
   return store_header(Header{kMagic, H.S.p_begin, H.S.n, H.S.nb, *kept, *vnnz, 0, 0}, x.header, record, s);
 }
 
@@ -1561,6 +1582,7 @@ Csr transposed_csr(const Csr& c, const TaskArrays& A, int64_t out_rows, int64_t 
 template <typename I>
 spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes, hipStream_t s,
                       spmm_taskmap_info* info, spmm_plan_record* record) {
+  Ends ends;
   const win::Matrix wm = window_matrix(c);
   if (window_task_eligible(c, graph_layout)) {
     const bool layout = graph_layout && c.rows == c.cols;
@@ -1592,6 +1614,7 @@ spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
       *info = r;
       return store_header(Header{kMagicWindows, v.p_begin, v.n, 0, 0, 0, 0, v.naic}, B.header, record, s);
     }
+    ends = ends_of(v);
   }
   Ctx x;
   TaskArrays A;
@@ -1601,7 +1624,7 @@ spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
   lay_task(x, A, c, layout, ws);
   if (x.arena.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
   WinSort& S = A.S;
-  if (spmm_status st = run_window_sort<I>(c, 16, false, S, x)) return st;
+  if (spmm_status st = run_window_sort<I>(c, 16, false, ends, S, x)) return st;
   const int64_t nwin = S.nwin, nb = S.nb, n = S.n;
 
   // Windows by density (descending), id ascending (custom_op.cpp:784-811).
@@ -1679,9 +1702,7 @@ spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
     // P * A^T * P^T: entry (r, c) goes to row inv[c], column inv[r], in
     // (row, position) order (packed_column_reindex.h:43-101), then the fixed
     // 295/505 split (pack_fixed_layout, custom_op.cpp:1350-1384).
-    int64_t last = 0;
-    if (spmm_status st = read_back(&last, S.row_first + c.rows, 1, s)) return st;
-    if (S.p_begin != 0 || S.p_begin + last != c.nnz)
+    if (S.p_begin != 0 || n != c.nnz)
       return fail(SPMM_ERR_INVALID_ARGUMENT, "CSR row pointer does not end at nnz");
     // Element ids and packed rows below 2^32 travel packed in the sort value.
     const int packed = n <= 0xFFFFFFFFll && hs.out_rows <= 0xFFFFFFFFll ? 1 : 0;
@@ -1699,7 +1720,8 @@ spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
     if (st) return st;
     const Csr t = transposed_csr(c, A, hs.out_rows, n);
     int64_t tk = 0, tv = 0;
-    if (spmm_status st2 = hybrid_run<int64_t>(t, 295.0 / 505.0, 16, A.T, x, &tk, &tv)) return st2;
+    // transpose_rowptr's pointer is monotone from 0 to n.
+    if (spmm_status st2 = hybrid_run<int64_t>(t, 295.0 / 505.0, 16, Ends{0, n}, A.T, x, &tk, &tv)) return st2;
     r.t_windows = A.T.S.nwin;
     r.t_blocks = tk;
     r.t_rows = A.T.S.nwin * 16;

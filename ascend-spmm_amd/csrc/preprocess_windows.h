@@ -23,6 +23,10 @@ struct Matrix {
 
 inline bool eligible(Op op, const Matrix& m, int64_t W) { return eligible(op, m.rows, m.cols, m.nnz, W); }
 
+// A plan's record holds p_begin and n, whatever else err says (not of a row
+// pointer that is not monotone inside [0, nnz]).
+bool ends_known(int64_t err);
+
 // Device record of a plan, read back by the host in one copy.
 struct WindowState {
   int64_t err;             // nonzero: not for this path (or an input error)

@@ -37,7 +37,21 @@ namespace {
 typedef unsigned int u2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int u4_t __attribute__((ext_vector_type(4)));
 
-enum : int { kGeneral = 1 };  // WindowState::err: take the sorting pipeline
+// A plan's error word: take the sorting pipeline; kBadRows: the row pointer
+// is not monotone inside [0, nnz].
+enum : unsigned long long { kGeneral = 1, kBadRows = 2 };
+
+// Raises err's bits (its kernel's other work-groups may read it meanwhile).
+__device__ inline void raise_error(int64_t* err, unsigned long long bits) {
+  atomicOr(reinterpret_cast<unsigned long long*>(err), bits);
+}
+// err at entry for a whole work-group, in an LDS word: one thread's load,
+// complete at the next barrier.  Wavefronts must not each read a word that
+// their own launch raises.
+__device__ inline void peek(const int64_t* err, uint32_t* stop) {
+  if (threadIdx.x == 64)  // not the wavefront that loads the window's rows
+    *stop = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ? 1u : 0u;
+}
 
 // ------------------------------------------------------------- bitmap sizes
 
@@ -100,6 +114,15 @@ __device__ inline void load_window(const P* __restrict__ rowptr, int64_t rows, i
     }
   }
   __syncthreads();
+}
+
+// The plan's first position and nonzeros, by the work-group of window 0.
+template <typename P, typename State>
+__device__ inline void load_ends(const P* __restrict__ rowptr, int64_t rows, State* st) {
+  if (threadIdx.x == 0) {
+    st->p_begin = static_cast<int64_t>(rowptr[0]);
+    st->n = static_cast<int64_t>(rowptr[rows]) - st->p_begin;
+  }
 }
 
 // The same in scalar registers: the LDS copy would be read again for every
@@ -406,15 +429,19 @@ __global__ __launch_bounds__(1024) void count_windows(const I* __restrict__ rowp
                                                       uint32_t* __restrict__ rank, State* __restrict__ st) {
   extern __shared__ __align__(16) uint32_t bm[];
   __shared__ WindowRows s;
-  __shared__ uint32_t s_count;
+  __shared__ uint32_t s_count, s_stop;
   const int64_t w = blockIdx.x;
+  peek(&st->err, &s_stop);
   clear_words(bm, words);
   if (threadIdx.x == 0) s_count = 0;
   load_window(rowptr, rows, nnz, w, W, &s);
+  if (w == 0) load_ends(rowptr, rows, st);
   uint32_t held[kHold];
   int bad = s.ok && !long_window(s.n, nnz) ? 0 : 1;
-  if (!bad) set_bits<true>(CsrColumns<I>{col}, RowStarts(s), cols, bm, held, &bad);  // uniform
-  if (bad) st->err = kGeneral;
+  // Once a window is bad the counts are of no use: the rest only leave values
+  // that the next kernels can go through.  Uniform.
+  if (!bad && !s_stop) set_bits<true>(CsrColumns<I>{col}, RowStarts(s), cols, bm, held, &bad);
+  if (bad) raise_error(&st->err, s.ok ? kGeneral : kGeneral | kBadRows);
   __syncthreads();
   uint32_t c = count_bits(bm, words);
   if ((threadIdx.x & 63) == 0 && c != 0) atomicAdd(&s_count, c);
@@ -434,10 +461,8 @@ __global__ __launch_bounds__(1024) void count_windows(const I* __restrict__ rowp
 // work-group, kScanPer windows per thread and round.
 constexpr int kScanPer = 8;
 
-template <typename I>
 __global__ __launch_bounds__(1024) void scan_windows(const uint32_t* __restrict__ nb, int64_t nwin,
-                                                     uint32_t* __restrict__ ptr, const I* __restrict__ rowptr,
-                                                     int64_t rows, WindowState* __restrict__ st) {
+                                                     uint32_t* __restrict__ ptr, WindowState* __restrict__ st) {
   __shared__ uint32_t s_wave[17];
   uint32_t carry = 0;
   for (int64_t i0 = 0; i0 < nwin; i0 += 1024 * kScanPer) {
@@ -457,8 +482,6 @@ __global__ __launch_bounds__(1024) void scan_windows(const uint32_t* __restrict_
   }
   if (threadIdx.x == 0) {
     ptr[nwin] = carry;
-    st->p_begin = static_cast<int64_t>(rowptr[0]);
-    st->n = static_cast<int64_t>(rowptr[rows]) - st->p_begin;
     st->total = carry;
   }
 }
@@ -761,11 +784,10 @@ __global__ __launch_bounds__(1024) void task_decide(const I* __restrict__ rowptr
   __shared__ int64_t s_q;
   __shared__ uint32_t s_bpos, h[17], cb[17], cn[17], s_rows[17];
   const uint32_t tid = threadIdx.x;
-  if (st->err != 0) return;  // uniform
-  const int64_t p_begin = static_cast<int64_t>(rowptr[0]);
-  const int64_t n = static_cast<int64_t>(rowptr[rows]) - p_begin;
+  if (st->err != 0) return;  // uniform, or every wavefront leaves below
+  const int64_t p_begin = st->p_begin, n = st->n;
   if (layout && (p_begin != 0 || n != nnz)) {
-    if (tid == 0) st->err = kGeneral;
+    if (tid == 0) raise_error(&st->err, kGeneral);
     return;
   }
   if (tid == 0) s_bpos = ~0u;
@@ -938,8 +960,6 @@ __global__ __launch_bounds__(1024) void task_decide(const I* __restrict__ rowptr
     const int64_t naic = none ? 0 : static_cast<int64_t>(s_bpos) + (q > 0 ? 1 : 0);
     const int64_t last_rows = rows - 16 * (nwin - 1);
     const int64_t aiv_rows = 16 * (nwin - naic) - (st->last_pos >= naic ? 16 - last_rows : 0);
-    st->p_begin = p_begin;
-    st->n = n;
     st->bpos = none ? -1 : static_cast<int64_t>(s_bpos);
     st->bwin = bwin;
     st->bblocks = c;
@@ -1228,31 +1248,34 @@ __device__ inline void count_occupancy(const Cols& cols_at, const RowStarts& s, 
 // Blocks per window by occupancy, and their sums over all windows (spread over
 // kHistCopies counters: same-address atomics run one after another).  `stop`
 // (or null) is an error word of earlier kernels, which makes this one leave;
-// it stores its own errors to `err`, a different word: were it the same one,
+// it raises its own errors in `err`, a different word: were it the same one,
 // the wavefronts of a work-group could read it before and after another
 // work-group's store, and those that stayed would use the LDS of those that
-// left, and write by it.
+// left, and write by it.  `ends` (or null) takes the first position and the
+// number of nonzeros.
 template <typename P, typename Cols, bool kCheck>
 __global__ __launch_bounds__(1024) void split_counts(const P* __restrict__ rowptr, Cols col, int64_t rows,
                                                      int64_t cols, int64_t nnz, int W, uint32_t words, uint32_t groups,
                                                      int gshift, uint32_t* __restrict__ nb, uint32_t* __restrict__ hist,
                                                      uint32_t* __restrict__ total, uint32_t* occ_far,
-                                                     const int64_t* stop, int64_t* err) {
+                                                     const int64_t* stop, int64_t* err, WindowState* ends) {
   extern __shared__ __align__(16) uint32_t bm[];
   uint32_t* const prefix = bm + words;
   __shared__ WindowRows s;
-  __shared__ uint32_t s_wave[17], s_hist[32];
+  __shared__ uint32_t s_wave[17], s_hist[32], s_stop;
   if (stop != nullptr && *stop != 0) return;  // uniform: not written in this launch
   const int64_t w = blockIdx.x;
+  peek(err, &s_stop);
   clear_words(bm, words);
   if (threadIdx.x < 32) s_hist[threadIdx.x] = 0u;
   load_window(rowptr, rows, nnz, w, W, &s);
+  if (ends != nullptr && w == 0) load_ends(rowptr, rows, ends);
   uint32_t held[kHold];
   int bad = s.ok && !long_window(s.n, nnz) ? 0 : 1;
   const RowStarts starts(s);
-  if (!bad) set_bits<kCheck>(col, starts, cols, bm, held, &bad);  // uniform
-  if (bad) *err = kGeneral;
-  if (__syncthreads_or(bad)) return;
+  if (!bad && !s_stop) set_bits<kCheck>(col, starts, cols, bm, held, &bad);  // uniform
+  if (bad) raise_error(err, s.ok ? kGeneral : kGeneral | kBadRows);
+  if (__syncthreads_or(bad || s_stop)) return;
   const uint32_t blocks = bitmap_prefix(bm, prefix, words, gshift, s_wave);
   const bool near = blocks <= kOccLds;
   uint32_t* const occ = near ? prefix + groups : occ_far + s.base;
@@ -1577,7 +1600,7 @@ spmm_status plan_blocks(const Matrix& m, int64_t W, bool tiles, const BlockArray
                        static_cast<const I*>(m.col), m.rows, m.cols, m.nnz, static_cast<int>(W), b.words, a.nb,
                        static_cast<uint64_t*>(nullptr), static_cast<uint32_t*>(nullptr),
                        static_cast<uint32_t*>(nullptr), a.state);
-    hipLaunchKernelGGL(scan_windows<I>, dim3(1), dim3(1024), 0, s, a.nb, nwin, a.ptr, rowptr, m.rows, a.state);
+    hipLaunchKernelGGL(scan_windows, dim3(1), dim3(1024), 0, s, a.nb, nwin, a.ptr, a.state);
     return check_launch("window counts");
   });
 }
@@ -1608,14 +1631,14 @@ namespace {
 
 template <typename P, typename Cols, bool kCheck>
 spmm_status run_split(const P* rowptr, Cols col, int64_t rows, int64_t cols, int64_t nnz, double a, int64_t W,
-                      const SplitArrays& x, const int64_t* stop, int64_t* err, int64_t* kept, int64_t* vnnz,
-                      hipStream_t s) {
+                      const SplitArrays& x, const int64_t* stop, int64_t* err, WindowState* ends, int64_t* kept,
+                      int64_t* vnnz, hipStream_t s) {
   const int64_t nwin = ceil_div(rows, W);
   const BitmapShape b(cols, nnz, nwin);
   const size_t lds = b.lds() + kOccLds * sizeof(uint32_t);
   hipLaunchKernelGGL((split_counts<P, Cols, kCheck>), dim3(static_cast<unsigned>(nwin)), dim3(b.threads(lds)), lds, s,
                      rowptr, col, rows, cols, nnz, static_cast<int>(W), b.words, b.groups, b.gshift, x.nb, x.hist,
-                     x.total, x.occ, stop, err);
+                     x.total, x.occ, stop, err, ends);
   hipLaunchKernelGGL(split_decide, dim3(1), dim3(1024), 0, s, nwin, a, x.nb, x.hist, x.total, x.moved, x.kptr, x.vptr,
                      x.rule, stop, static_cast<const int64_t*>(err), kept, vnnz);
   return check_launch("split counts");
@@ -1642,7 +1665,7 @@ spmm_status plan_split(const Matrix& m, double a, int64_t W, const SplitArrays& 
     init_state(state, x.total, 16 * kHistCopies, s);
     return run_split<I, CsrColumns<I>, true>(static_cast<const I*>(m.rowptr),
                                              CsrColumns<I>{static_cast<const I*>(m.col)}, m.rows, m.cols, m.nnz, a, W,
-                                             x, nullptr, &state->err, &state->total, &state->vnnz, s);
+                                             x, nullptr, &state->err, state, &state->total, &state->vnnz, s);
   });
 }
 
@@ -1671,6 +1694,8 @@ int key_bits(uint64_t max_value) {
 }
 
 }  // namespace
+
+bool ends_known(int64_t err) { return (err & static_cast<int64_t>(kBadRows)) == 0; }
 
 size_t task_temp_bytes(const Matrix& m, bool layout) {
   size_t a = 0, b = 0;
@@ -1736,7 +1761,7 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, hipStre
                        x.stkey, m.nnz, 16 * nwin, x.record, x.rp);
     return run_split<uint32_t, WordColumns, false>(x.rp, WordColumns{x.stword}, 16 * nwin, 16 * nwin, m.nnz,
                                                    295.0 / 505.0, 16, x.split, &x.record->err, &x.record->t_err,
-                                                   &x.record->t_kept, &x.record->t_vnnz, s);
+                                                   nullptr, &x.record->t_kept, &x.record->t_vnnz, s);
   });
 }
 

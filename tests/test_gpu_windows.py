@@ -178,6 +178,44 @@ def test_longest_window(spmm_npu, n):
     assert_same(spmm_npu.preprocess(*gpu(*args), 3, 40000), O.preprocess(*args, 3, 40000))
 
 
+@pytest.mark.parametrize("first", [0, 11])
+def test_handed_over_matrices_keep_their_first_position(spmm_npu, first):
+    """The sorting pipeline takes a handed-over matrix's first position and
+    nonzeros from the window plan: row pointers that start past zero, and end
+    before the last stored nonzero, with a repeated column."""
+    crow, col = square(500)
+    r = int(np.nonzero(np.diff(crow) > 3)[0][5])
+    col = col.copy()
+    col[crow[r] + 1] = col[crow[r]]
+    crow, col = crow + first, np.concatenate([np.arange(first), col, np.arange(7)])
+    args = as_types(crow, col, np.int32, np.float32)
+    assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 500, 500, 16), O.csr_to_bcsr(*args, 500, 500, 16))
+    assert_same(spmm_npu.csr_to_ascend_cube(*gpu(*args), 500, 500, 16), O.csr_to_ascend_cube(*args, 500, 500, 16))
+    assert_same(spmm_npu.block_level_split(*gpu(*args), 500, 500, 0.6, 16),
+                O.block_level_split(*args, 500, 500, 0.6, 16))
+    assert_same(spmm_npu.preprocess(*gpu(*args), 500, 500), O.preprocess(*args, 500, 500))
+    with pytest.raises(ValueError, match="end at nnz"):
+        spmm_npu.preprocess(*gpu(*args), 500, 500, graph_layout=True)
+
+
+@pytest.mark.parametrize("unsorted", [False, True])
+def test_row_pointers_that_decrease_are_refused(spmm_npu, unsorted):
+    """Also where another window's columns alone hand the matrix over."""
+    crow, col = square(700)
+    if unsorted:
+        col = col[::-1].copy()
+    back = crow.copy()
+    back[651], back[650] = crow[650], crow[651]
+    args = gpu(*as_types(back, col, np.int32, np.float32))
+    for call in (lambda: spmm_npu.csr_to_bcsr(*args, 700, 700, 16),
+                 lambda: spmm_npu.csr_to_ascend_cube(*args, 700, 700, 16),
+                 lambda: spmm_npu.block_level_split(*args, 700, 700, 0.6, 16),
+                 lambda: spmm_npu.preprocess(*args, 700, 700),
+                 lambda: spmm_npu.preprocess(*args, 700, 700, graph_layout=True)):
+        with pytest.raises(ValueError, match="row pointer"):
+            call()
+
+
 def hub_column(n, hub, seed=4):
     """Short rows, the first `hub` of which hold column 7 too."""
     rng = np.random.default_rng(seed)
