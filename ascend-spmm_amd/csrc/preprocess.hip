@@ -1588,10 +1588,11 @@ spmm_status task_plan(const Csr& c, bool graph_layout, void* ws, size_t ws_bytes
     const bool layout = graph_layout && c.rows == c.cols;
     const WindowTask B(c, layout, ws);
     if (B.used > ws_bytes) return fail(SPMM_ERR_CONTRACT, "preprocessing workspace too small");
-    if (spmm_status st = win::plan_task(wm, layout, B.x, s)) return st;
+    bool handed_over = false;
+    if (spmm_status st = win::plan_task(wm, layout, B.x, &handed_over, s)) return st;
     win::TaskRecord v;
     if (spmm_status st = read_back(&v, B.x.record, 1, s)) return st;
-    if (v.err == 0 && v.t_err == 0) {
+    if (!handed_over && v.err == 0 && v.t_err == 0) {
       spmm_taskmap_info r{};
       r.aic_windows = v.naic;
       r.aic_blocks = v.aic_blocks;

@@ -97,7 +97,9 @@ struct TaskArrays {
 
 // Temporary bytes of the device sorts.
 size_t task_temp_bytes(const Matrix& m, bool layout);
-spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, hipStream_t s);
+// handed_over: the counts have found the matrix not to be for this pipeline,
+// and the plan has ended there.
+spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, bool* handed_over, hipStream_t s);
 // naic: the plan's TaskRecord::naic.
 spmm_status fill_task(const Matrix& m, bool layout, int64_t naic, const TaskArrays& x, const spmm_taskmap_out* o,
                       hipStream_t s);

@@ -41,10 +41,12 @@ typedef unsigned int u4_t __attribute__((ext_vector_type(4)));
 // is not monotone inside [0, nnz].
 enum : unsigned long long { kGeneral = 1, kBadRows = 2 };
 
-// Raises err's bits (its kernel's other work-groups may read it meanwhile).
+// Raises err's bits (its kernel's other work-groups may read it meanwhile); by
+// one thread of a work-group, as same-address atomics run one after another.
 __device__ inline void raise_error(int64_t* err, unsigned long long bits) {
   atomicOr(reinterpret_cast<unsigned long long*>(err), bits);
 }
+
 // err at entry for a whole work-group, in an LDS word: one thread's load,
 // complete at the next barrier.  Wavefronts must not each read a word that
 // their own launch raises.
@@ -429,11 +431,11 @@ __global__ __launch_bounds__(1024) void count_windows(const I* __restrict__ rowp
                                                       uint32_t* __restrict__ rank, State* __restrict__ st) {
   extern __shared__ __align__(16) uint32_t bm[];
   __shared__ WindowRows s;
-  __shared__ uint32_t s_count, s_stop;
+  __shared__ uint32_t s_count, s_stop, s_bad;
   const int64_t w = blockIdx.x;
   peek(&st->err, &s_stop);
   clear_words(bm, words);
-  if (threadIdx.x == 0) s_count = 0;
+  if (threadIdx.x == 0) s_count = s_bad = 0;
   load_window(rowptr, rows, nnz, w, W, &s);
   if (w == 0) load_ends(rowptr, rows, st);
   uint32_t held[kHold];
@@ -441,12 +443,13 @@ __global__ __launch_bounds__(1024) void count_windows(const I* __restrict__ rowp
   // Once a window is bad the counts are of no use: the rest only leave values
   // that the next kernels can go through.  Uniform.
   if (!bad && !s_stop) set_bits<true>(CsrColumns<I>{col}, RowStarts(s), cols, bm, held, &bad);
-  if (bad) raise_error(&st->err, s.ok ? kGeneral : kGeneral | kBadRows);
+  if (bad) s_bad = 1;
   __syncthreads();
   uint32_t c = count_bits(bm, words);
   if ((threadIdx.x & 63) == 0 && c != 0) atomicAdd(&s_count, c);
   __syncthreads();
   if (threadIdx.x == 0) {
+    if (s_bad) raise_error(&st->err, s.ok ? kGeneral : kGeneral | kBadRows);
     nb[w] = kTiles ? (s_count + 15u) / 16u : s_count;
     if (dkey != nullptr) {
       const double density = s_count ? static_cast<double>(s.n) / static_cast<double>(s_count) : 0.0;
@@ -758,6 +761,7 @@ __global__ __launch_bounds__(256) void place_windows(const uint32_t* __restrict_
 // then first nonzero, so the nonzeros of the first q blocks follow from the
 // 16 occupancy counts, and only the boundary occupancy's blocks need their
 // first nonzeros ranked: no sort.
+// host_err (or null): a host word that takes the plan's errors so far.
 constexpr int kDecidePer = 8;
 
 // blocks / 295 >= nonzeros / 505 in double precision (custom_op.cpp:813-826).
@@ -776,7 +780,8 @@ __global__ __launch_bounds__(1024) void task_decide(const I* __restrict__ rowptr
                                                     const uint32_t* __restrict__ nb, const uint32_t* __restrict__ swin,
                                                     const uint64_t* __restrict__ sbz, uint32_t* pnb, uint32_t* pnnz,
                                                     uint32_t near_blocks, uint32_t* far_occ, uint32_t* far_first,
-                                                    uint32_t* midx, uint32_t* mrow, TaskRecord* st) {
+                                                    uint32_t* midx, uint32_t* mrow, TaskRecord* st,
+                                                    int64_t* host_err) {
   extern __shared__ __align__(16) uint32_t bm[];
   uint32_t* const prefix = bm + words;
   __shared__ WindowRows s;
@@ -784,12 +789,16 @@ __global__ __launch_bounds__(1024) void task_decide(const I* __restrict__ rowptr
   __shared__ int64_t s_q;
   __shared__ uint32_t s_bpos, h[17], cb[17], cn[17], s_rows[17];
   const uint32_t tid = threadIdx.x;
-  if (st->err != 0) return;  // uniform, or every wavefront leaves below
   const int64_t p_begin = st->p_begin, n = st->n;
-  if (layout && (p_begin != 0 || n != nnz)) {
-    if (tid == 0) raise_error(&st->err, kGeneral);
-    return;
+  const bool part = layout && (p_begin != 0 || n != nnz);
+  const int64_t err = st->err;  // raised below only: a wavefront that reads it then leaves as well
+  if (tid == 0) {
+    if (part) raise_error(&st->err, kGeneral);
+    if (host_err != nullptr)
+      __hip_atomic_store(host_err, part ? static_cast<int64_t>(kGeneral) : err, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
   }
+  if (part || err != 0) return;  // uniform
   if (tid == 0) s_bpos = ~0u;
   uint32_t carry_b = 0, carry_z = 0;  // blocks, nonzeros
   __syncthreads();
@@ -1265,7 +1274,7 @@ __global__ __launch_bounds__(1024) void split_counts(const P* __restrict__ rowpt
   __shared__ uint32_t s_wave[17], s_hist[32], s_stop;
   if (stop != nullptr && *stop != 0) return;  // uniform: not written in this launch
   const int64_t w = blockIdx.x;
-  peek(err, &s_stop);
+  if (kCheck) peek(err, &s_stop);  // the transpose's errors are a few long windows
   clear_words(bm, words);
   if (threadIdx.x < 32) s_hist[threadIdx.x] = 0u;
   load_window(rowptr, rows, nnz, w, W, &s);
@@ -1273,9 +1282,12 @@ __global__ __launch_bounds__(1024) void split_counts(const P* __restrict__ rowpt
   uint32_t held[kHold];
   int bad = s.ok && !long_window(s.n, nnz) ? 0 : 1;
   const RowStarts starts(s);
-  if (!bad && !s_stop) set_bits<kCheck>(col, starts, cols, bm, held, &bad);  // uniform
-  if (bad) raise_error(err, s.ok ? kGeneral : kGeneral | kBadRows);
-  if (__syncthreads_or(bad || s_stop)) return;
+  if (!bad && !(kCheck && s_stop)) set_bits<kCheck>(col, starts, cols, bm, held, &bad);  // uniform
+  if (__syncthreads_or(bad)) {
+    if (threadIdx.x == 0) raise_error(err, s.ok ? kGeneral : kGeneral | kBadRows);
+    return;
+  }
+  if (kCheck && s_stop) return;
   const uint32_t blocks = bitmap_prefix(bm, prefix, words, gshift, s_wave);
   const bool near = blocks <= kOccLds;
   uint32_t* const occ = near ? prefix + groups : occ_far + s.base;
@@ -1697,6 +1709,60 @@ int key_bits(uint64_t max_value) {
 
 bool ends_known(int64_t err) { return (err & static_cast<int64_t>(kBadRows)) == 0; }
 
+namespace {
+
+// A pinned word per host thread, freed when the thread ends.
+struct HostWord {
+  int64_t* p = nullptr;
+  ~HostWord() {
+    if (p != nullptr) (void)hipHostFree(p);
+  }
+  int64_t* get() {
+    if (p == nullptr &&
+        hipHostMalloc(reinterpret_cast<void**>(&p), sizeof *p, hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+    }
+    return p;
+  }
+};
+thread_local HostWord host_word;
+
+// A value that a kernel of this call stores to the thread's word, which the
+// host looks at while the stream goes on.
+struct Verdict {
+  static constexpr int64_t kPending = -1;
+  int64_t* word;
+  hipStream_t stream;
+  bool due = false;  // the store has been launched and not been seen
+  Verdict(bool wanted, hipStream_t s) : word(wanted ? host_word.get() : nullptr), stream(s) {
+    if (word != nullptr) __atomic_store_n(word, kPending, __ATOMIC_SEQ_CST);
+  }
+  // The stored value; 0 without a word, or once the stream has run dry.
+  spmm_status wait(int64_t* value) {
+    *value = 0;
+    if (!due) return SPMM_OK;
+    for (uint32_t looks = 1;; ++looks) {
+      int64_t v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+      if (v == kPending && looks % 65536 == 0) {
+        const hipError_t e = hipStreamQuery(stream);
+        if (e != hipSuccess && e != hipErrorNotReady) return check_hip(e, "waiting for the counts");
+        if (e == hipSuccess && (v = __atomic_load_n(word, __ATOMIC_ACQUIRE)) == kPending) v = 0;
+      }
+      if (v != kPending) {
+        due = false;
+        *value = v;
+        return SPMM_OK;
+      }
+    }
+  }
+  ~Verdict() {  // after an error: no store may come once the word serves another call
+    if (due) (void)hipStreamSynchronize(stream);
+  }
+};
+
+}  // namespace
+
 size_t task_temp_bytes(const Matrix& m, bool layout) {
   size_t a = 0, b = 0;
   const size_t nwin = static_cast<size_t>(ceil_div(m.rows, 16));
@@ -1709,8 +1775,14 @@ size_t task_temp_bytes(const Matrix& m, bool layout) {
   return a > b ? a : b;
 }
 
-spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, hipStream_t s) {
+spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, bool* handed_over, hipStream_t s) {
+  *handed_over = false;
   const int64_t nwin = ceil_div(m.rows, 16);
+  // The sort of the transposed entries, a fifth of the plan, is not started for
+  // a matrix that the counts hand over: task_decide first stores their verdict
+  // to a host word, and the host launches the sort while the GPU is still at
+  // work on the rest of task_decide.
+  Verdict verdict(layout, s);
   const BitmapShape b(m.cols, m.nnz, nwin);
   return by_index(m.index_type, [&](auto i) {
     using I = decltype(i);
@@ -1738,8 +1810,9 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, hipStre
         b.lds() <= 100 * 1024 ? static_cast<uint32_t>((152 * 1024 - b.lds()) / (3 * sizeof(uint32_t)) / 4 * 4) : 0;
     hipLaunchKernelGGL(task_decide<I>, dim3(1), dim3(1024), b.lds() + 3 * near_blocks * sizeof(uint32_t), s, rowptr, col, m.rows, m.cols, m.nnz, nwin,
                        b.words, b.groups, b.gshift, layout ? 1 : 0, x.nb, x.swin, x.sbz, x.pnb, x.pnnz, near_blocks, x.mocc, x.mfirst,
-                       x.midx, x.mrow, x.record);
+                       x.midx, x.mrow, x.record, verdict.word);
     if (spmm_status st = check_launch("task mapping")) return st;
+    verdict.due = verdict.word != nullptr;
     if (!layout) return SPMM_OK;
     // P A^T P^T and its fixed 295/505 split.
     hipLaunchKernelGGL(task_inverse, dim3(static_cast<unsigned>(ceil_div(16 * nwin, 256))), dim3(256), 0, s, x.swin,
@@ -1751,6 +1824,12 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, hipStre
           return check_launch("transpose keys");
         }))
       return st;
+    int64_t err = 0;
+    if (spmm_status st = verdict.wait(&err)) return st;
+    if (err != 0) {
+      *handed_over = true;
+      return SPMM_OK;
+    }
     bytes = x.temp_bytes;
     if (hipError_t e = rocprim::radix_sort_pairs(x.temp, bytes, static_cast<const uint32_t*>(x.tkey), x.stkey,
                                                  static_cast<const uint64_t*>(x.tword), x.stword,

@@ -3,6 +3,8 @@ behaviour (bitmap word and prefix-group edges, windows longer than the
 registers hold, the LDS tile's edge, the column limit), bit for bit against
 the CPU oracle; and the inputs they hand to the sorting pipeline instead."""
 
+import concurrent.futures
+
 import numpy as np
 import pytest
 import torch
@@ -196,6 +198,34 @@ def test_handed_over_matrices_keep_their_first_position(spmm_npu, first):
     assert_same(spmm_npu.preprocess(*gpu(*args), 500, 500), O.preprocess(*args, 500, 500))
     with pytest.raises(ValueError, match="end at nnz"):
         spmm_npu.preprocess(*gpu(*args), 500, 500, graph_layout=True)
+
+
+def test_graph_plans_of_several_threads_and_streams(spmm_npu):
+    """The counts' verdict reaches the host in a word of its own per thread:
+    four threads with a stream each, matrices that are handed over and others
+    in turn."""
+    plans = []
+    for n, turned in ((333, False), (334, True), (1601, False), (1602, True)):
+        crow, col = square(n)
+        if turned:
+            col = np.concatenate([col[a:b][::-1] for a, b in zip(crow, crow[1:])])
+        args = as_types(crow, col, np.int32, np.float32)
+        plans.append((n, gpu(*args), O.preprocess(*args, n, n, graph_layout=True)))
+    torch.cuda.synchronize()
+
+    def work(t):
+        stream, out = torch.cuda.Stream(), []
+        with torch.cuda.stream(stream):
+            for i in range(12):
+                n, args, _ = plans[(t + i) % 4]
+                out.append(spmm_npu.preprocess(*args, n, n, graph_layout=True))
+        stream.synchronize()
+        return out
+
+    with concurrent.futures.ThreadPoolExecutor(4) as pool:
+        for t, out in enumerate(pool.map(work, range(4))):
+            for i, got in enumerate(out):
+                assert_same(got, plans[(t + i) % 4][2])
 
 
 @pytest.mark.parametrize("unsorted", [False, True])
