@@ -72,11 +72,6 @@ constexpr int kStageUnroll = 18;
 #ifndef SPMM_GATHER_SPLIT_BYTES
 #define SPMM_GATHER_SPLIT_BYTES 512
 #endif
-// Column pieces of one cache line (gather_typed says when).
-constexpr int64_t kLineBytes = 128;
-constexpr int64_t kL2Bytes = int64_t(4) << 20;  // one XCD's
-constexpr int64_t kLineReuse = 8;       // nonzeros per dense row, at least
-constexpr int64_t kLineMaxDegree = 64;  // nonzeros per row, at most
 // A row is "short" (summed by one lane group, never split) when it holds at
 // most short_max(R) nonzeros: R / 2, or all of R for ranges of at most
 // SPMM_GATHER_SHORT_FULL positions, where a lane group that runs on past its
@@ -1446,14 +1441,21 @@ spmm_status gather_typed(const void* rowptr, const void* col, const void* value,
   while ((1 << log2L) < lanes_needed && log2L < 6) ++log2L;
   int L = 1 << log2L;
   int64_t chunks = ceil_div(lanes_needed, L);
-  // Dense operands within a 32-bit byte extent use buffer loads.
-  const int64_t extent = buffer_extent(K, ld, N, sizeof(T));
-  const bool buffer = extent <= kBufferLimit;
-  const bool seg_sizes = g.cwin == 0 && g.nnz >= kSegMinNnz && K > 0 && buffer && extent <= kSegMaxDenseBytes;
   // Dense rows of at least SPMM_GATHER_SPLIT_BYTES: one work-group per
   // column chunk of a tile (rows of one chunk are halved first), so
   // neighbouring work-groups, which run on different XCDs, gather different
   // column pieces and each XCD's L2 holds a fraction of the dense operand.
+  //
+  // More parts (128-byte pieces, up to one part per XCD) help where gathers
+  // miss the L2s and cost where they hit, as every part stages the tile's
+  // nonzeros anew, and sizes do not tell which.  With this split / eight parts,
+  // us, rows of 1 KB unless said: spmm_csr on 60000 uniform rows of 16
+  // 135 / 107, 30000 of 32 111 / 69, 50000 power-law rows of 20 142 / 112, a
+  // graph's training step (131072 rows of 30) 1551 / 1442; but on a 27-point
+  // stencil of 32^3 50.5 / 62.2, a 9-point one of 256^2 47.1 / 55.4 (30.0 /
+  // 33.4 at 512 bytes), a band of 16 over 50000 rows 41.9 / 53.4, 50000 rows
+  // half of them in 16x16 blocks 66 / 77; in the mixed operator a 27-point
+  // stencil of 40^3 87 / 99.
   int wg_split = 1;
   if (SPMM_GATHER_SPLIT_BYTES > 0 && N * static_cast<int64_t>(sizeof(T)) >= SPMM_GATHER_SPLIT_BYTES) {
     if (chunks == 1 && L >= 16 && lanes_needed == L) {
@@ -1462,37 +1464,6 @@ spmm_status gather_typed(const void* rowptr, const void* col, const void* value,
       chunks = 2;
     }
     wg_split = static_cast<int>(chunks);  // 2: lanes_needed <= 128 and L = 64 for the widest rows
-  }
-  // Cache-line pieces (kLineBytes, up to one part per XCD) where the gathers
-  // are likely to miss the L2s: each XCD then reads an eighth of the columns
-  // and its 4 MB L2 holds eight times as many dense rows.  The matrix is not
-  // read to find out, so the line is drawn by sizes.  Against the split above
-  // (us; fp32 rows of 1 KB unless said): spmm_csr on 50000 power-law rows of
-  // 20, 143 -> 112, on 30000 uniform rows of 32 (fp16), 112 -> 68, 60000
-  // uniform rows of 16 at 256-byte rows, 37.5 -> 31.4; a graph's training
-  // step (131072 rows of 30), 1558 -> 1444.  Every part stages the tile's
-  // nonzeros anew, so it does not pay
-  //  * where a dense row is gathered a few times only (kLineReuse): half
-  //    blocked, half scattered, 3 per dense row at 1 KB, 175 -> 197;
-  //  * for long rows (kLineMaxDegree; in the mixed operator the rows after
-  //    the block windows, or all where every window has blocks), mostly
-  //    banded or clustered matrices, whose gathers hit the L2s anyway: a band
-  //    of 220 per row, 146 -> 314;
-  //  * with segment work-groups, which serve the long rows from a column slab
-  //    per XCD already: 100000 power-law rows of 20, 131 -> 146;
-  //  * for a dense operand that one L2 holds whole.
-  // Sizes do not show that rows of a window share columns: spmm_csr on 50000
-  // rows, half of them in 16x16 blocks, takes 77 us for 65.
-  const int64_t row_bytes = N * static_cast<int64_t>(sizeof(T));
-  const int64_t free_rows = vrows > 16 * g.cwin ? vrows - 16 * g.cwin : vrows;
-  if (!seg_sizes && chunks == wg_split && lanes_needed == L * chunks && row_bytes >= 2 * kLineBytes &&
-      extent > kL2Bytes && g.nnz >= kLineReuse * K && g.nnz <= kLineMaxDegree * free_rows) {
-    while (L * 16 > kLineBytes && chunks < kXcds) {
-      --log2L;
-      L >>= 1;
-      chunks *= 2;
-    }
-    wg_split = static_cast<int>(chunks);
   }
   int64_t ranges_per_tile = (kWgThreads / L) / (chunks / wg_split);
   if (ranges_per_tile > kTileRanges) ranges_per_tile = kTileRanges;
@@ -1535,6 +1506,9 @@ spmm_status gather_typed(const void* rowptr, const void* col, const void* value,
   g.tail = static_cast<int64_t*>(ws);
   float* partial = reinterpret_cast<float*>(static_cast<char*>(ws) + tail_bytes);
 
+  // Dense operands within a 32-bit byte extent use buffer loads.
+  const int64_t extent = buffer_extent(K, ld, N, sizeof(T));
+  const bool buffer = extent <= kBufferLimit;
   // Segment work-groups for spmm_csr on large matrices whose dense operand
   // is at most kSegMaxDenseBytes (an XCD's column slab of it then stays near
   // its L2).  The vector part of the mixed operator holds the rows the cost
@@ -1554,7 +1528,8 @@ spmm_status gather_typed(const void* rowptr, const void* col, const void* value,
   g.tile_shift = log2_of(ranges_per_tile * g.range);
   const bool pow2 = (int64_t(1) << g.seg_chunk_log2) == g.seg_chunk && (int64_t(1) << g.range_log2) == g.range &&
                     (int64_t(1) << g.tile_shift) == ranges_per_tile * g.range;
-  const bool seg_on = seg_sizes && wg_threads % 64 == 0 && pow2;
+  const bool seg_on = g.cwin == 0 && g.nnz >= kSegMinNnz && K > 0 && buffer && extent <= kSegMaxDenseBytes &&
+                      wg_threads % 64 == 0 && pow2;
   g.seg = seg_on ? reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + tail_bytes + partial_bytes) : nullptr;
   g.seg_flag = seg_on ? reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + tail_bytes + partial_bytes + seg_bytes)
                       : nullptr;

@@ -400,20 +400,18 @@ def test_vector_path_width_invariant_bitwise(spmm_npu, dtype):
 @pytest.mark.parametrize("dtype,width", [("fp16", 128), ("fp16", 256), ("fp16", 512), ("fp16", 1024),
                                          ("fp32", 64), ("fp32", 128), ("fp32", 512)])
 @pytest.mark.parametrize("mixed", [False, True])
-def test_line_pieces_equal_narrow_rows_bitwise(spmm_npu, dtype, width, mixed):
-    """Rows of 8 to 64 nonzeros over a dense operand larger than one L2 take
-    column pieces of one cache line; C[:, :16], C[:, 16:32], ... computed alone
-    (dense rows too narrow for them) are the same bits.  Long rows cross ranges
-    and tiles, some columns are invalid, the row count is ragged, and in the
-    mixed operator one block window takes vector sums."""
+def test_column_parts_equal_narrow_rows_bitwise(spmm_npu, dtype, width, mixed):
+    """Dense rows of 512 bytes or more go to column parts on separate
+    work-groups; C[:, :16], C[:, 16:32], ... computed alone (rows too narrow
+    for them) are the same bits.  Long rows cross ranges and tiles, some
+    columns are invalid, the row count is ragged, and in the mixed operator one
+    block window takes vector sums."""
     rng = np.random.default_rng(311)
     rows, cols = 16_411, 17_000
     crow, col = random_csr(rng, rows, cols, 25, long_rows=[(5, 900), (8000, 3000), (rows - 1, 700)])
-    assert cols * 8 <= col.size <= rows * 64
     col[[0, col.size // 2, col.size - 1]] = [cols, -1, cols + 7]
     vals = rng.uniform(-1, 1, col.size).astype(NP_DT[dtype])
     B = rng.standard_normal((cols, width)).astype(NP_DT[dtype])
-    assert B.nbytes > 4 << 20
 
     def run(b):
         if not mixed:
