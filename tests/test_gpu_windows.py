@@ -66,14 +66,27 @@ def test_tile_edge(spmm_npu, blocks, value, extra):
     assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 2, 5000, 16), O.csr_to_bcsr(*args, 2, 5000, 16))
 
 
-@pytest.mark.parametrize("n", [4095, 4096, 4097])
-def test_window_of_register_size(spmm_npu, n):
-    """A window of as many nonzeros as a 256-thread work-group holds."""
+@pytest.mark.parametrize("threads,cols,others", [(256, 3000, 12), (512, 3000, 0), (1024, 1 << 20, 0)])
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_window_of_register_size(spmm_npu, threads, cols, others, extra):
+    """A window of as many nonzeros as a work-group's threads hold in registers
+    (8 each), one less, one more.  Work-groups have 256 threads where the
+    windows average at most 1024 nonzeros (here among `others` short ones), 512
+    where they hold more, and 1024 beside a bitmap that fills the LDS."""
+    n = 8 * threads + extra
     rng = np.random.default_rng(n)
-    rows = [np.sort(rng.choice(3000, k, replace=False)) for k in (1500, n - 3000, 1500)]
+    rows = [np.sort(rng.choice(cols, k, replace=False)) for k in (n // 3, n - 2 * (n // 3), n // 3)]
+    rows += [np.zeros(0, np.int64)] * 13
+    for _ in range(16 * others):
+        rows.append(np.sort(rng.choice(cols, 5, replace=False)))
+    mean = sum(r.size for r in rows) // (1 + others)
+    assert (mean <= 1024) == (others > 0)
     crow = np.concatenate([[0], np.cumsum([r.size for r in rows])]).astype(np.int64)
     args = as_types(crow, np.concatenate(rows).astype(np.int64), np.int32, np.float16)
-    assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), 3, 3000, 16), O.csr_to_bcsr(*args, 3, 3000, 16))
+    assert_same(spmm_npu.csr_to_bcsr(*gpu(*args), len(rows), cols, 16), O.csr_to_bcsr(*args, len(rows), cols, 16))
+    assert_same(spmm_npu.block_level_split(*gpu(*args), len(rows), cols, 0.6, 16),
+                O.block_level_split(*args, len(rows), cols, 0.6, 16))
+    assert_same(spmm_npu.preprocess(*gpu(*args), len(rows), cols), O.preprocess(*args, len(rows), cols))
 
 
 def test_first_position_past_zero(spmm_npu):
