@@ -1090,7 +1090,8 @@ spmm_status run_window_sort(const Csr& c, int64_t W, bool check_sorted, const En
            S.row_of, S.col64, check_sorted ? 1 : 0, S.err);
   launch(window_keys, S.n, s, S.row_of, S.col64, S.n, W, c.cols, S.key, S.elem);
   if (spmm_status st = check_launch("window_keys")) return st;
-  const uint64_t maxkey = static_cast<uint64_t>(S.nwin > 0 ? S.nwin : 1) * static_cast<uint64_t>(c.cols > 0 ? c.cols : 1);
+  const uint64_t maxkey =
+      static_cast<uint64_t>(S.nwin > 0 ? S.nwin : 1) * static_cast<uint64_t>(c.cols > 0 ? c.cols : 1);
   if (hipError_t e = x.prims.sort_pairs(S.key, S.skey, S.elem, S.selem, S.n, bits_for(maxkey)))
     return check_hip(e, "window sort");
   launch(run_heads, S.n, s, S.skey, S.n, S.head);

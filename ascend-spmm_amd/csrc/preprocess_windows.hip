@@ -13,15 +13,20 @@
 // 1380 us there, 144 us here: counting 30 us, writing 78 us, the read-back
 // that sizes the outputs and launches the rest; preprocess of 2.0M power-law
 // nonzeros 762 -> 150 us, of a 7.2M-nonzero graph with its packed transpose
-// 4079 -> 1114 us).  The splits need no sort of the blocks either: they take
+// 4079 -> 1117 us).  The splits need no sort of the blocks either: they take
 // blocks in order of occupancy, then first nonzero, so counts per occupancy
 // give every prefix, and only one window's blocks of one occupancy are ranked.
 //
 // Bound: vector instructions per nonzero on long windows (about 130 in
-// write_blocks, 60 in count_windows), and on short ones the latency of a
-// window's steps (row pointers, columns, LDS atomics, scan), which the other
-// windows resident on the CU cover: a bitmap of 100,000 columns is 12.5 KB,
-// and work-groups are sized so that a CU holds 1024-2048 threads of them.
+// write_blocks, 60 in count_windows).  On short ones each window's own cost:
+// the latency of its steps (row pointers, columns, LDS atomics, scan), which the
+// other windows resident on the CU cover, and the clears and sweeps of its
+// bitmap, one word per 32 columns however few nonzeros there are.  At 262,144
+// columns a window of 480 nonzeros clears 8192 words in every kernel and sweeps
+// them once to count and twice to rank, about as many wavefront instructions as
+// its nonzeros take.  Past some width the sorting pipeline is the faster one
+// (window_rule.h).  Work-groups are sized so that a CU holds 1024-2048 threads
+// of them: a bitmap of 100,000 columns is 12.5 KB.
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include <algorithm>
@@ -210,7 +215,9 @@ __device__ inline V block_exclusive(V v, V* s_wave, V* sum) {
 // wavefront takes consecutive quads of words, 64 at a time, so that its reads
 // meet no bank conflict: a first sweep counts its bits, a second one writes
 // the counts before each group.
-__device__ inline uint32_t quad_bits(const u4_t& b) { return __popc(b[0]) + __popc(b[1]) + __popc(b[2]) + __popc(b[3]); }
+__device__ inline uint32_t quad_bits(const u4_t& b) {
+  return __popc(b[0]) + __popc(b[1]) + __popc(b[2]) + __popc(b[3]);
+}
 
 __device__ inline uint32_t bitmap_prefix(const uint32_t* bm, uint32_t* prefix, uint32_t words, int gshift,
                                          uint32_t* s_wave) {
@@ -527,7 +534,9 @@ struct ValueTile {
   uint32_t* col;  // [kBlocks]: the blocks' columns
   __device__ inline explicit ValueTile(uint32_t* lds) : p(reinterpret_cast<Unit*>(lds)), col(lds + kTileBytes / 4) {}
   static constexpr size_t kLds = kTileBytes + kBlocks * sizeof(uint32_t);
-  __device__ inline uint32_t unit(uint32_t b, uint32_t j) const { return b * kUnits + ((j + (b >> kShift)) & (kUnits - 1)); }
+  __device__ inline uint32_t unit(uint32_t b, uint32_t j) const {
+    return b * kUnits + ((j + (b >> kShift)) & (kUnits - 1));
+  }
   __device__ inline void set(uint32_t b, uint32_t rr, U v) const {
     reinterpret_cast<U*>(p)[unit(b, rr / kPerUnit) * kPerUnit + rr % kPerUnit] = v;
   }
@@ -547,7 +556,8 @@ template <bool kTiles, typename I, typename U>
 __device__ inline void emit_blocks(const WindowRows& s, const I* __restrict__ col, const U* __restrict__ val,
                                    int64_t cols, uint32_t* bm, uint32_t words, uint32_t groups, int gshift,
                                    uint32_t* s_wave, uint32_t tile_blocks, uint32_t blocks, I* __restrict__ uniq,
-                                   U* __restrict__ out, const uint32_t* __restrict__ packed, I* __restrict__ renumbered) {
+                                   U* __restrict__ out, const uint32_t* __restrict__ packed,
+                                   I* __restrict__ renumbered) {
   uint32_t* const prefix = bm + words;
   constexpr int64_t kUnit = kTiles ? 256 : 16;  // values per block or tile
   // Windows whose blocks fit the LDS tile are put together there; longer ones
@@ -615,7 +625,8 @@ __device__ inline void emit_blocks(const WindowRows& s, const I* __restrict__ co
           const uint32_t rr = starts.row(i);
           uniq[b] = static_cast<I>(held[k]);
           if (packed != nullptr) renumbered[b] = static_cast<I>(packed[starts.base + i]);
-          out[kTiles ? 256 * static_cast<int64_t>(b / 16) + 16 * rr + b % 16 : 16 * static_cast<int64_t>(b) + rr] = v[k];
+          out[kTiles ? 256 * static_cast<int64_t>(b / 16) + 16 * rr + b % 16 : 16 * static_cast<int64_t>(b) + rr] =
+              v[k];
         }
       }
     }
@@ -646,7 +657,8 @@ __global__ __launch_bounds__(1024) void write_blocks(const I* __restrict__ rowpt
     if (w == nwin - 1) crow[nwin] = static_cast<I>(p1);
   }
   emit_blocks<kTiles>(s, col, val, cols, bm, words, groups, gshift, s_wave, tile_blocks, p1 - p0,
-                      uniq + (kTiles ? 16 : 1) * static_cast<int64_t>(p0), out + (kTiles ? 256 : 16) * static_cast<int64_t>(p0),
+                      uniq + (kTiles ? 16 : 1) * static_cast<int64_t>(p0),
+                      out + (kTiles ? 256 : 16) * static_cast<int64_t>(p0),
                       static_cast<const uint32_t*>(nullptr), static_cast<I*>(nullptr));
 }
 
@@ -688,8 +700,8 @@ __device__ inline uint32_t window_nnz(const P* __restrict__ rowptr, int64_t rows
 // sbz[position] = blocks << 32 | nonzeros.
 //
 // rank_windows counts, for 64 windows per wavefront, those that come before
-// each among a sixteenth of the keys, which it loads 64 at a time and hands
-// round by lane reads; place_windows writes the windows to their ranks.
+// each among 64 * kRankBlocks of the keys, which it loads 64 at a time and
+// hands round by lane reads; place_windows writes the windows to their ranks.
 // nwin^2 comparisons, but two launches; past kRankWindows windows the device
 // radix sort takes over (six launches, 33 us for 6250 windows) and
 // place_windows only fetches the pairs.  Fetching them here spreads the
@@ -837,7 +849,8 @@ __global__ __launch_bounds__(1024) void task_decide(const I* __restrict__ rowptr
         pnnz[a + k] = pz;
         pb += b[k];
         pz += z[k];
-        if (found == ~0u && block_cost_reaches(pb, nnz - static_cast<int64_t>(pz))) found = static_cast<uint32_t>(a + k);
+        if (found == ~0u && block_cost_reaches(pb, nnz - static_cast<int64_t>(pz)))
+          found = static_cast<uint32_t>(a + k);
       }
     }
     if (found != ~0u) atomicMin(&s_bpos, found);
@@ -1119,7 +1132,8 @@ __global__ __launch_bounds__(1024) void write_block_rows(const I* __restrict__ r
   I* const runiq = packed != nullptr ? static_cast<I*>(o.runiq) + p0 : nullptr;
   U* const out = static_cast<U*>(o.val) + 16 * p0;
   if (!split) {
-    emit_blocks<false>(s, col, val, cols, bm, words, groups, gshift, s_wave, tile_blocks, nb[w], uniq, out, packed, runiq);
+    emit_blocks<false>(s, col, val, cols, bm, words, groups, gshift, s_wave, tile_blocks, nb[w], uniq, out, packed,
+                       runiq);
     return;
   }
   // The marginal window, shared by both parts: kept blocks at midx, the other
@@ -1449,11 +1463,11 @@ __global__ __launch_bounds__(1024) void split_decide(int64_t nwin, double a,
 
 // A window's outputs of the split.
 template <typename P, typename Cols, typename Vals, typename O, typename U>
-__global__ __launch_bounds__(1024) void write_split(const P* __restrict__ rowptr, Cols cols_at, Vals vals_at, int64_t rows,
-                                                    int64_t cols, int64_t nnz, int W, int64_t nwin, uint32_t words,
-                                                    uint32_t groups, int gshift, SplitArrays x, O* __restrict__ crow,
-                                                    O* __restrict__ uniq, U* __restrict__ out, O* __restrict__ vrow,
-                                                    O* __restrict__ vcol, U* __restrict__ vval) {
+__global__ __launch_bounds__(1024) void write_split(const P* __restrict__ rowptr, Cols cols_at, Vals vals_at,
+                                                    int64_t rows, int64_t cols, int64_t nnz, int W, int64_t nwin,
+                                                    uint32_t words, uint32_t groups, int gshift, SplitArrays x,
+                                                    O* __restrict__ crow, O* __restrict__ uniq, U* __restrict__ out,
+                                                    O* __restrict__ vrow, O* __restrict__ vcol, U* __restrict__ vval) {
   extern __shared__ __align__(16) uint32_t bm[];
   uint32_t* const prefix = bm + words;
   __shared__ WindowRows s;
@@ -1663,9 +1677,10 @@ spmm_status launch_split_fill(const P* rowptr, Cols col, Vals val, int64_t rows,
   const int64_t nwin = ceil_div(rows, W);
   const BitmapShape b(cols, nnz, nwin);
   const size_t lds = b.lds() + kOccLds * sizeof(uint32_t);
-  hipLaunchKernelGGL((write_split<P, Cols, Vals, O, U>), dim3(static_cast<unsigned>(nwin)), dim3(b.threads(lds)), lds, s, rowptr, col, val, rows, cols, nnz, static_cast<int>(W),
-                     nwin, b.words, b.groups, b.gshift, x, static_cast<O*>(crow), static_cast<O*>(uniq), out,
-                     static_cast<O*>(vrow), static_cast<O*>(vcol), vval);
+  hipLaunchKernelGGL((write_split<P, Cols, Vals, O, U>), dim3(static_cast<unsigned>(nwin)), dim3(b.threads(lds)), lds,
+                     s, rowptr, col, val, rows, cols, nnz, static_cast<int>(W), nwin, b.words, b.groups, b.gshift, x,
+                     static_cast<O*>(crow), static_cast<O*>(uniq), out, static_cast<O*>(vrow), static_cast<O*>(vcol),
+                     vval);
   return check_launch("split outputs");
 }
 
@@ -1789,15 +1804,19 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, bool* h
     const I* rowptr = static_cast<const I*>(m.rowptr);
     const I* col = static_cast<const I*>(m.col);
     init_state(x.record, layout ? x.split.total : nullptr, layout ? 16 * kHistCopies : 0, s);
+    const size_t count_lds = b.words * sizeof(uint32_t);
     hipLaunchKernelGGL((count_windows<I, false, TaskRecord>), dim3(static_cast<unsigned>(nwin)),
-                       dim3(b.threads(b.words * sizeof(uint32_t))), b.words * sizeof(uint32_t), s, rowptr, col, m.rows, m.cols, m.nnz, 16, b.words, x.nb, x.dkey,
-                       x.wid, x.rank, x.record);
+                       dim3(b.threads(count_lds)), count_lds, s, rowptr, col, m.rows, m.cols, m.nnz, 16, b.words, x.nb,
+                       x.dkey, x.wid, x.rank, x.record);
     if (spmm_status st = check_launch("window counts")) return st;
     size_t bytes = x.temp_bytes;
     const bool ranked = nwin <= kRankWindows;
     if (ranked) {
-      hipLaunchKernelGGL(rank_windows, dim3(static_cast<unsigned>(ceil_div(nwin, 64)), static_cast<unsigned>(ceil_div(ceil_div(nwin, 64), kRankBlocks))), dim3(64), 0, s,
-                         x.dkey, nwin, x.rank);
+      const int64_t key_blocks = ceil_div(nwin, 64);
+      hipLaunchKernelGGL(rank_windows,
+                         dim3(static_cast<unsigned>(key_blocks),
+                              static_cast<unsigned>(ceil_div(key_blocks, kRankBlocks))),
+                         dim3(64), 0, s, x.dkey, nwin, x.rank);
     } else if (hipError_t e = rocprim::radix_sort_pairs(x.temp, bytes, static_cast<const uint64_t*>(x.dkey), x.sdkey,
                                                         static_cast<const uint32_t*>(x.wid), x.swin,
                                                         static_cast<size_t>(nwin), 0, 64, s)) {
@@ -1808,9 +1827,9 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, bool* h
                        x.sbz, x.record);
     const uint32_t near_blocks =
         b.lds() <= 100 * 1024 ? static_cast<uint32_t>((152 * 1024 - b.lds()) / (3 * sizeof(uint32_t)) / 4 * 4) : 0;
-    hipLaunchKernelGGL(task_decide<I>, dim3(1), dim3(1024), b.lds() + 3 * near_blocks * sizeof(uint32_t), s, rowptr, col, m.rows, m.cols, m.nnz, nwin,
-                       b.words, b.groups, b.gshift, layout ? 1 : 0, x.nb, x.swin, x.sbz, x.pnb, x.pnnz, near_blocks, x.mocc, x.mfirst,
-                       x.midx, x.mrow, x.record, verdict.word);
+    hipLaunchKernelGGL(task_decide<I>, dim3(1), dim3(1024), b.lds() + 3 * near_blocks * sizeof(uint32_t), s, rowptr,
+                       col, m.rows, m.cols, m.nnz, nwin, b.words, b.groups, b.gshift, layout ? 1 : 0, x.nb, x.swin,
+                       x.sbz, x.pnb, x.pnnz, near_blocks, x.mocc, x.mfirst, x.midx, x.mrow, x.record, verdict.word);
     if (spmm_status st = check_launch("task mapping")) return st;
     verdict.due = verdict.word != nullptr;
     if (!layout) return SPMM_OK;

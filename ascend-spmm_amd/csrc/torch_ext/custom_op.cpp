@@ -520,8 +520,9 @@ std::map<std::string, at::Tensor> preprocess(at::Tensor crow_ptr, at::Tensor col
   at::Tensor ws = workspace(d.crow, ws_bytes);
   spmm_taskmap_info info;
   spmm_plan_record plan;
-  raise_status(spmm_taskmap_plan_record(&m, window_size, graph_layout ? 1 : 0, ws.data_ptr(), ws_bytes, s, &info, &plan),
-               "preprocess");
+  raise_status(
+      spmm_taskmap_plan_record(&m, window_size, graph_layout ? 1 : 0, ws.data_ptr(), ws_bytes, s, &info, &plan),
+      "preprocess");
   const bool layout = info.packed_layout_supported != 0;
   std::map<std::string, at::Tensor> out;
   out["crow_window_ptr"] = idx_tensor(d, info.aic_windows + 1);
