@@ -52,12 +52,21 @@ __device__ inline void raise_error(int64_t* err, unsigned long long bits) {
   atomicOr(reinterpret_cast<unsigned long long*>(err), bits);
 }
 
-// err at entry for a whole work-group, in an LDS word: one thread's load,
-// complete at the next barrier.  Wavefronts must not each read a word that
-// their own launch raises.
-__device__ inline void peek(const int64_t* err, uint32_t* stop) {
-  if (threadIdx.x == 64)  // not the wavefront that loads the window's rows
-    *stop = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ? 1u : 0u;
+// Plan kernels, at entry, by a thread outside the wavefront that loads the
+// window's rows: the plan's first position and nonzeros (window 0; ends may be
+// null), and *stop, an LDS word complete at the next barrier: whether err is
+// raised already.  One thread reads it, as wavefronts must not each read a word
+// that their own launch raises, and only in grids of more work-groups than run
+// at once (a load past the L2s: 0.6 us of a conversion of 42).
+template <typename P, typename State>
+__device__ inline void enter_plan(const P* __restrict__ rowptr, int64_t rows, State* ends, const int64_t* err,
+                                  uint32_t* stop) {
+  if (threadIdx.x != 64) return;
+  *stop = gridDim.x > 4096 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ? 1u : 0u;
+  if (blockIdx.x == 0 && ends != nullptr) {
+    ends->p_begin = static_cast<int64_t>(rowptr[0]);
+    ends->n = static_cast<int64_t>(rowptr[rows]) - static_cast<int64_t>(rowptr[0]);
+  }
 }
 
 // ------------------------------------------------------------- bitmap sizes
@@ -121,15 +130,6 @@ __device__ inline void load_window(const P* __restrict__ rowptr, int64_t rows, i
     }
   }
   __syncthreads();
-}
-
-// The plan's first position and nonzeros, by the work-group of window 0.
-template <typename P, typename State>
-__device__ inline void load_ends(const P* __restrict__ rowptr, int64_t rows, State* st) {
-  if (threadIdx.x == 0) {
-    st->p_begin = static_cast<int64_t>(rowptr[0]);
-    st->n = static_cast<int64_t>(rowptr[rows]) - st->p_begin;
-  }
 }
 
 // The same in scalar registers: the LDS copy would be read again for every
@@ -440,11 +440,10 @@ __global__ __launch_bounds__(1024) void count_windows(const I* __restrict__ rowp
   __shared__ WindowRows s;
   __shared__ uint32_t s_count, s_stop, s_bad;
   const int64_t w = blockIdx.x;
-  peek(&st->err, &s_stop);
+  enter_plan(rowptr, rows, st, &st->err, &s_stop);
   clear_words(bm, words);
   if (threadIdx.x == 0) s_count = s_bad = 0;
   load_window(rowptr, rows, nnz, w, W, &s);
-  if (w == 0) load_ends(rowptr, rows, st);
   uint32_t held[kHold];
   int bad = s.ok && !long_window(s.n, nnz) ? 0 : 1;
   // Once a window is bad the counts are of no use: the rest only leave values
@@ -1288,11 +1287,10 @@ __global__ __launch_bounds__(1024) void split_counts(const P* __restrict__ rowpt
   __shared__ uint32_t s_wave[17], s_hist[32], s_stop;
   if (stop != nullptr && *stop != 0) return;  // uniform: not written in this launch
   const int64_t w = blockIdx.x;
-  if (kCheck) peek(err, &s_stop);  // the transpose's errors are a few long windows
+  if (kCheck) enter_plan(rowptr, rows, ends, err, &s_stop);  // the transpose's errors are a few long windows
   clear_words(bm, words);
   if (threadIdx.x < 32) s_hist[threadIdx.x] = 0u;
   load_window(rowptr, rows, nnz, w, W, &s);
-  if (ends != nullptr && w == 0) load_ends(rowptr, rows, ends);
   uint32_t held[kHold];
   int bad = s.ok && !long_window(s.n, nnz) ? 0 : 1;
   const RowStarts starts(s);
@@ -1734,7 +1732,8 @@ struct HostWord {
   }
   int64_t* get() {
     if (p == nullptr &&
-        hipHostMalloc(reinterpret_cast<void**>(&p), sizeof *p, hipHostMallocPortable) != hipSuccess) {
+        hipHostMalloc(reinterpret_cast<void**>(&p), sizeof *p, hipHostMallocPortable | hipHostMallocCoherent) !=
+            hipSuccess) {
       (void)hipGetLastError();
       p = nullptr;
     }
@@ -1759,7 +1758,9 @@ struct Verdict {
     if (!due) return SPMM_OK;
     for (uint32_t looks = 1;; ++looks) {
       int64_t v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
-      if (v == kPending && looks % 65536 == 0) {
+      // Rarely, tenths of a second apart: the query puts a marker in the stream
+      // (6 us between two kernels).
+      if (v == kPending && looks % (1u << 27) == 0) {
         const hipError_t e = hipStreamQuery(stream);
         if (e != hipSuccess && e != hipErrorNotReady) return check_hip(e, "waiting for the counts");
         if (e == hipSuccess && (v = __atomic_load_n(word, __ATOMIC_ACQUIRE)) == kPending) v = 0;
