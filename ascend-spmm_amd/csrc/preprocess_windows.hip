@@ -10,10 +10,10 @@
 // ids are read twice, the values once, and no per-nonzero array is ever
 // written, where the sorting pipeline moves about 20 words of 8 bytes per
 // nonzero through memory (csr_to_bcsr of 14.4M nonzeros in 4096 banded windows:
-// 1380 us there, 144 us here: counting 30 us, writing 78 us, the read-back
+// 1380 us there, 148 us here: counting 31 us, writing 85 us, the read-back
 // that sizes the outputs and launches the rest; preprocess of 2.0M power-law
-// nonzeros 762 -> 150 us, of a 7.2M-nonzero graph with its packed transpose
-// 4079 -> 1117 us).  The splits need no sort of the blocks either: they take
+// nonzeros 762 -> 146 us, of a 7.2M-nonzero graph with its packed transpose
+// 4079 -> 1109 us).  The splits need no sort of the blocks either: they take
 // blocks in order of occupancy, then first nonzero, so counts per occupancy
 // give every prefix, and only one window's blocks of one occupancy are ranked.
 //
