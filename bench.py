@@ -74,28 +74,28 @@ OP_KERNELS = {
 FETCH_SCALE = 2.0
 WRITE_SCALE = 1.0
 PMC_KIB = {
-    (2, "csr", 128): {"fetch_kib": 151664.0, "write_kib": 32708.3, "sources": "113fc3377585db2c",
+    (2, "csr", 128): {"fetch_kib": 151508.0, "write_kib": 32708.4, "sources": "daaba2f603f9a93a",
                       "profile": "profiles/gather_c2_csr_n128_traffic.md"},
-    (3, "mixed", 128): {"fetch_kib": 95199.2, "write_kib": 28595.1, "sources": "113fc3377585db2c",
+    (3, "mixed", 128): {"fetch_kib": 95180.2, "write_kib": 28594.9, "sources": "daaba2f603f9a93a",
                         "profile": "profiles/mixed_c3_n128_traffic.md"},
-    (3, "bcsr", 128): {"fetch_kib": 35790.3, "write_kib": 16384.0, "sources": "113fc3377585db2c",
+    (3, "bcsr", 128): {"fetch_kib": 35786.9, "write_kib": 16384.0, "sources": "daaba2f603f9a93a",
                        "profile": "profiles/block_c3_bcsr_n128_traffic.md"},
-    (3, "bcsr", 256): {"fetch_kib": 47033.9, "write_kib": 32768.0, "sources": "113fc3377585db2c",
+    (3, "bcsr", 256): {"fetch_kib": 47015.7, "write_kib": 32768.0, "sources": "daaba2f603f9a93a",
                        "profile": "profiles/block_c3_bcsr_n256_traffic.md"},
-    (4, "mixed", 512): {"fetch_kib": 409029.1, "write_kib": 209044.9, "sources": "113fc3377585db2c",
+    (4, "mixed", 512): {"fetch_kib": 409017.1, "write_kib": 209043.7, "sources": "daaba2f603f9a93a",
                         "profile": "profiles/mixed_c4_n512_traffic.md"},
-    (1, "csr", 128): {"fetch_kib": 15795.3, "write_kib": 8256.0, "sources": "113fc3377585db2c",
+    (1, "csr", 128): {"fetch_kib": 15794.8, "write_kib": 8256.0, "sources": "daaba2f603f9a93a",
                       "profile": "profiles/gather_c1_csr_n128_traffic.md"},
-    (3, "csr", 128): {"fetch_kib": 98295.3, "write_kib": 73071.9, "sources": "113fc3377585db2c",
+    (3, "csr", 128): {"fetch_kib": 98293.6, "write_kib": 73072.0, "sources": "daaba2f603f9a93a",
                       "profile": "profiles/gather_c3_csr_n128_traffic.md"},
-    (3, "mixed", 256): {"fetch_kib": 165836.2, "write_kib": 56965.8, "sources": "113fc3377585db2c",
+    (3, "mixed", 256): {"fetch_kib": 165510.6, "write_kib": 56965.9, "sources": "daaba2f603f9a93a",
                         "profile": "profiles/mixed_c3_n256_traffic.md"},
-    (4, "mixed", 64): {"fetch_kib": 56335.0, "write_kib": 26255.0, "sources": "113fc3377585db2c",
+    (4, "mixed", 64): {"fetch_kib": 56334.8, "write_kib": 26255.0, "sources": "daaba2f603f9a93a",
                        "profile": "profiles/mixed_c4_n64_traffic.md"},
     # Per call: the op's kernels times their dispatches per call (four column
     # passes of gather_tiles, gather_post and block_windows; gather_rows for P
     # and for P^T; scatter_inverse and fill_minus_one once).
-    (5, "graph", 512): {"fetch_kib": 36690259.8, "write_kib": 7052596.5, "sources": "113fc3377585db2c",
+    (5, "graph", 512): {"fetch_kib": 36686769.1, "write_kib": 7052603.2, "sources": "daaba2f603f9a93a",
                         "profile": "profiles/graph_c5_n512_traffic.md"},
 }
 
