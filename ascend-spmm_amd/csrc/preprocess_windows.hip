@@ -1744,12 +1744,12 @@ thread_local HostWord host_word;
 
 // A value that a kernel of this call stores to the thread's word, which the
 // host looks at while the stream goes on.
-struct Verdict {
+struct Awaited {
   static constexpr int64_t kPending = -1;
   int64_t* word;
   hipStream_t stream;
   bool due = false;  // the store has been launched and not been seen
-  Verdict(bool wanted, hipStream_t s) : word(wanted ? host_word.get() : nullptr), stream(s) {
+  Awaited(bool wanted, hipStream_t s) : word(wanted ? host_word.get() : nullptr), stream(s) {
     if (word != nullptr) __atomic_store_n(word, kPending, __ATOMIC_SEQ_CST);
   }
   // The stored value; 0 without a word, or once the stream has run dry.
@@ -1772,7 +1772,7 @@ struct Verdict {
       }
     }
   }
-  ~Verdict() {  // after an error: no store may come once the word serves another call
+  ~Awaited() {  // after an error: no store may come once the word serves another call
     if (due) (void)hipStreamSynchronize(stream);
   }
 };
@@ -1795,10 +1795,10 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, bool* h
   *handed_over = false;
   const int64_t nwin = ceil_div(m.rows, 16);
   // The sort of the transposed entries, a fifth of the plan, is not started for
-  // a matrix that the counts hand over: task_decide first stores their verdict
-  // to a host word, and the host launches the sort while the GPU is still at
+  // a matrix that the counts hand over: task_decide first stores their error
+  // word to a host word, and the host launches the sort while the GPU is still at
   // work on the rest of task_decide.
-  Verdict verdict(layout, s);
+  Awaited counts_err(layout, s);
   const BitmapShape b(m.cols, m.nnz, nwin);
   return by_index(m.index_type, [&](auto i) {
     using I = decltype(i);
@@ -1830,9 +1830,9 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, bool* h
         b.lds() <= 100 * 1024 ? static_cast<uint32_t>((152 * 1024 - b.lds()) / (3 * sizeof(uint32_t)) / 4 * 4) : 0;
     hipLaunchKernelGGL(task_decide<I>, dim3(1), dim3(1024), b.lds() + 3 * near_blocks * sizeof(uint32_t), s, rowptr,
                        col, m.rows, m.cols, m.nnz, nwin, b.words, b.groups, b.gshift, layout ? 1 : 0, x.nb, x.swin,
-                       x.sbz, x.pnb, x.pnnz, near_blocks, x.mocc, x.mfirst, x.midx, x.mrow, x.record, verdict.word);
+                       x.sbz, x.pnb, x.pnnz, near_blocks, x.mocc, x.mfirst, x.midx, x.mrow, x.record, counts_err.word);
     if (spmm_status st = check_launch("task mapping")) return st;
-    verdict.due = verdict.word != nullptr;
+    counts_err.due = counts_err.word != nullptr;
     if (!layout) return SPMM_OK;
     // P A^T P^T and its fixed 295/505 split.
     hipLaunchKernelGGL(task_inverse, dim3(static_cast<unsigned>(ceil_div(16 * nwin, 256))), dim3(256), 0, s, x.swin,
@@ -1845,7 +1845,7 @@ spmm_status plan_task(const Matrix& m, bool layout, const TaskArrays& x, bool* h
         }))
       return st;
     int64_t err = 0;
-    if (spmm_status st = verdict.wait(&err)) return st;
+    if (spmm_status st = counts_err.wait(&err)) return st;
     if (err != 0) {
       *handed_over = true;
       return SPMM_OK;

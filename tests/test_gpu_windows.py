@@ -214,7 +214,7 @@ def test_handed_over_matrices_keep_their_first_position(spmm_npu, first):
 
 
 def test_graph_plans_of_several_threads_and_streams(spmm_npu):
-    """The counts' verdict reaches the host in a word of its own per thread:
+    """The counts' error word reaches the host in a word of its own per thread:
     four threads with a stream each, matrices that are handed over and others
     in turn."""
     plans = []
