@@ -74,28 +74,28 @@ OP_KERNELS = {
 FETCH_SCALE = 2.0
 WRITE_SCALE = 1.0
 PMC_KIB = {
-    (2, "csr", 128): {"fetch_kib": 151508.0, "write_kib": 32708.4, "sources": "daaba2f603f9a93a",
+    (2, "csr", 128): {"fetch_kib": 151504.5, "write_kib": 32708.4, "sources": "520e37681ebe00dd",
                       "profile": "profiles/gather_c2_csr_n128_traffic.md"},
-    (3, "mixed", 128): {"fetch_kib": 95180.2, "write_kib": 28594.9, "sources": "daaba2f603f9a93a",
+    (3, "mixed", 128): {"fetch_kib": 95175.5, "write_kib": 28594.9, "sources": "520e37681ebe00dd",
                         "profile": "profiles/mixed_c3_n128_traffic.md"},
-    (3, "bcsr", 128): {"fetch_kib": 35786.9, "write_kib": 16384.0, "sources": "daaba2f603f9a93a",
+    (3, "bcsr", 128): {"fetch_kib": 35782.3, "write_kib": 16384.0, "sources": "520e37681ebe00dd",
                        "profile": "profiles/block_c3_bcsr_n128_traffic.md"},
-    (3, "bcsr", 256): {"fetch_kib": 47015.7, "write_kib": 32768.0, "sources": "daaba2f603f9a93a",
+    (3, "bcsr", 256): {"fetch_kib": 47016.1, "write_kib": 32768.0, "sources": "520e37681ebe00dd",
                        "profile": "profiles/block_c3_bcsr_n256_traffic.md"},
-    (4, "mixed", 512): {"fetch_kib": 409017.1, "write_kib": 209043.7, "sources": "daaba2f603f9a93a",
+    (4, "mixed", 512): {"fetch_kib": 408991.8, "write_kib": 209043.6, "sources": "520e37681ebe00dd",
                         "profile": "profiles/mixed_c4_n512_traffic.md"},
-    (1, "csr", 128): {"fetch_kib": 15794.8, "write_kib": 8256.0, "sources": "daaba2f603f9a93a",
+    (1, "csr", 128): {"fetch_kib": 15795.2, "write_kib": 8256.0, "sources": "520e37681ebe00dd",
                       "profile": "profiles/gather_c1_csr_n128_traffic.md"},
-    (3, "csr", 128): {"fetch_kib": 98293.6, "write_kib": 73072.0, "sources": "daaba2f603f9a93a",
+    (3, "csr", 128): {"fetch_kib": 98293.3, "write_kib": 73072.0, "sources": "520e37681ebe00dd",
                       "profile": "profiles/gather_c3_csr_n128_traffic.md"},
-    (3, "mixed", 256): {"fetch_kib": 165510.6, "write_kib": 56965.9, "sources": "daaba2f603f9a93a",
+    (3, "mixed", 256): {"fetch_kib": 165869.7, "write_kib": 56964.6, "sources": "520e37681ebe00dd",
                         "profile": "profiles/mixed_c3_n256_traffic.md"},
-    (4, "mixed", 64): {"fetch_kib": 56334.8, "write_kib": 26255.0, "sources": "daaba2f603f9a93a",
+    (4, "mixed", 64): {"fetch_kib": 56328.4, "write_kib": 26255.0, "sources": "520e37681ebe00dd",
                        "profile": "profiles/mixed_c4_n64_traffic.md"},
     # Per call: the op's kernels times their dispatches per call (four column
     # passes of gather_tiles, gather_post and block_windows; gather_rows for P
     # and for P^T; scatter_inverse and fill_minus_one once).
-    (5, "graph", 512): {"fetch_kib": 36686769.1, "write_kib": 7052603.2, "sources": "daaba2f603f9a93a",
+    (5, "graph", 512): {"fetch_kib": 36686090.9, "write_kib": 7052604.4, "sources": "520e37681ebe00dd",
                         "profile": "profiles/graph_c5_n512_traffic.md"},
 }
 
